@@ -455,17 +455,14 @@ void qlinearconv_impl(Backend* b, const dw_hip_buffer* input, const dw_hip_buffe
     if (wpk_bytes > sp.wpk_cap)
       dw::fail(DW_ERR_UNSUPPORTED, "qlinearconv: packed weights of " + std::to_string(wpk_bytes) +
                                        " bytes exceed the no-alloc scratch's " + std::to_string(sp.wpk_cap));
-    dw::launch_pack_weights(b->stream, kernel->ptr, sp.wpk, (int)(g.kh * g.kw * g.ci), (int)g.co, a.cout_pad,
-                            a.ksteps, 1);
-    a.wpk = (const uint8_t*)sp.wpk;
   } else {
-    a.wpk = (const uint8_t*)pack_into_ws(b, kernel, a, g, 1);
+    sp.wpk = b->workspace(Backend::WS_WPACK, wpk_bytes);
     sp.ms = (float*)b->workspace(Backend::WS_SCALE, c_out * 4);
     sp.bi = (int*)b->workspace(Backend::WS_BIAS, c_out * 4);
   }
-  b->upload_async(sp.ms, m_host, c_out * 4);
-  dw::launch_qconv_bias(b->stream, (const int8_t*)kernel->ptr, bias ? (const int*)bias->ptr : nullptr,
-                        sp.bi, (int)(k_h * k_w * c_in), (int)c_out, 128 - x_zp);
+  a.wpk = (const uint8_t*)sp.wpk;
+  dw::launch_qconv_prep(b->stream, kernel->ptr, sp.wpk, bias ? (const int*)bias->ptr : nullptr, sp.bi, sp.ms, m_host,
+                        (int)(k_h * k_w * c_in), (int)c_out, a.cout_pad, a.ksteps, 128 - x_zp);
   a.epi = dw::EPI_QU8;
   a.xxor = 0x80808080u;
   const uint32_t pb = (uint32_t)((x_zp ^ 0x80) & 0xff);

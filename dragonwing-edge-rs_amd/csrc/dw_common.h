@@ -246,9 +246,11 @@ struct DwArgs {
 // Packs HWIO weights (esize 1 or 2) into [ksteps][cout_pad][64B] rows.
 void launch_pack_weights(hipStream_t st, const void* w_hwio, void* wpk, int K, int cout,
                          int cout_pad, int ksteps, int esize);
-// bias_out[c] = (bias ? bias[c] : 0) + corr * sum_k w[k][c]   (int64 checked on host)
-void launch_qconv_bias(hipStream_t st, const int8_t* w_hwio, const int* bias, int* bias_out, int K,
-                       int cout, int corr);
+// The same for a QLinearConv's int8 weights, with its per-channel values:
+// bias_out[c] = (bias ? bias[c] : 0) + corr * sum_k w[k][c] (int32, wrapping)
+// and ms_out[c] = m_host[c], which is read before the call returns.
+void launch_qconv_prep(hipStream_t st, const void* w_hwio, void* wpk, const int* bias, int* bias_out, float* ms_out,
+                       const float* m_host, int K, int cout, int cout_pad, int ksteps, int corr);
 // Implicit-GEMM convolution; selects a tile shape for the problem.
 void launch_igemm(hipStream_t st, const IgemmArgs& a, int esize);
 // Two chained 3x3 QLinearConvs (c -> c -> c, c = 16, 32 or 64, stride 1,

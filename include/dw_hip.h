@@ -181,8 +181,8 @@ int dw_hip_qlinearconv_u8s8(dw_hip_backend* be, const dw_hip_buffer* input,
  * dw_hip_qlinearconv_u8s8.  Every call on a device shares that device's
  * scratch; calls through different backends (streams) on one device are
  * ordered on it (each call's stream waits for the previous call's last
- * launch).  Not capturable: the per-channel scales are copied from the
- * caller's host array and the call waits for that copy. */
+ * launch).  Not capturable: that order rests on an event recorded outside
+ * any capture.  The scales are read before the call returns. */
 int dw_hip_qlinearconv_u8s8_noalloc(dw_hip_backend* be, const dw_hip_buffer* input,
                                     const dw_hip_buffer* kernel, const dw_hip_buffer* bias,
                                     dw_hip_buffer* output, size_t n, size_t h_in, size_t w_in,
