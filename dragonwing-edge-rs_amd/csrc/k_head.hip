@@ -148,22 +148,36 @@ __global__ __launch_bounds__(256) void gemm_i8_kernel(const int8_t* A, const int
 // onnx runtime.rs:1109-1175): thread (batch, channel) sums its h x w values
 // in row-major order in f32 and divides by h * w (correctly rounded); f16
 // widens with the reference decode and rounds the mean to f16.
+// The sum is one ordered chain, so what counts is the loads in flight: 16 are
+// issued before the first is added (past the end the last value again, not
+// added), and workgroups of one wave spread a small batch over the CUs.
+// 32 x 7 x 7 x 1280 f32: 6.9-13.6 us before, 5.0 us.
+constexpr int kGapAhead = 16;
 template <bool F16>
-__global__ __launch_bounds__(256) void global_avg_pool_kernel(const void* X, void* Y, int n, int hw, int c) {
-  const int ch = blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(64) void global_avg_pool_kernel(const void* X, void* Y, int n, int hw, int c) {
+  using E = std::conditional_t<F16, uint16_t, float>;
+  const int ch = blockIdx.x * 64 + threadIdx.x;
   const int b = blockIdx.y;
   if (ch >= c || b >= n) return;
+  const E* x = (const E*)X + (size_t)b * hw * c + ch;
   float sum = 0.0f;
-  const size_t base = (size_t)b * hw * c + ch;
-  if constexpr (F16) {
-    const uint16_t* x = (const uint16_t*)X + base;
-    for (int s = 0; s < hw; ++s) sum += h2f(x[(size_t)s * c]);
-    ((uint16_t*)Y)[(size_t)b * c + ch] = f2h(__fdiv_rn(sum, (float)hw));
-  } else {
-    const float* x = (const float*)X + base;
-    for (int s = 0; s < hw; ++s) sum += x[(size_t)s * c];
-    ((float*)Y)[(size_t)b * c + ch] = __fdiv_rn(sum, (float)hw);
+  for (unsigned s0 = 0; s0 < (unsigned)hw; s0 += kGapAhead) {
+    E v[kGapAhead];
+#pragma unroll
+    for (int j = 0; j < kGapAhead; ++j) v[j] = x[(size_t)umin(s0 + j, hw - 1) * c];
+#pragma unroll
+    for (int j = 0; j < kGapAhead; ++j) {
+      float f;
+      if constexpr (F16) f = h2f(v[j]);
+      else f = v[j];
+      sum = s0 + j < (unsigned)hw ? sum + f : sum;
+    }
   }
+  const float mean = __fdiv_rn(sum, (float)hw);
+  if constexpr (F16)
+    ((uint16_t*)Y)[(size_t)b * c + ch] = f2h(mean);
+  else
+    ((float*)Y)[(size_t)b * c + ch] = mean;
 }
 
 // Reductions over a group of G consecutive threads (G = 16, 64: lanes of a
@@ -240,21 +254,66 @@ __global__ __launch_bounds__(256) void softmax_rows_kernel(const void* X, void* 
   }
 }
 
-// QLinearGlobalAveragePool over NHWC u8: thread (batch, channel) sums its
-// h x w values minus the input zero point as an int32, then
+// QLinearGlobalAveragePool over NHWC u8: per (batch, channel) the h x w
+// values minus the input zero point are summed as an int32, then
 // y = clamp(rint((float)sum * M) + y_zp, 0, 255) with M = (x_scale / y_scale)
 // / (h * w) in f32 (rint: round half to even).
+__device__ __forceinline__ uint8_t qgap_out(int acc, float m, int y_zp) {
+  const float q = rintf((float)acc * m) + (float)y_zp;
+  return (uint8_t)fminf(fmaxf(q, 0.0f), 255.0f);
+}
+
+// A workgroup owns 64 * 4 bytes of channels (a dword of four channels a lane,
+// c % 4 == 0) of one image; its four waves take a quarter of the pixels each,
+// kGapAhead loads in flight, and the sums (integers, any order) meet in LDS.
+// 32 x 7 x 7 x 1280: 7.1 us for a byte a thread walking all pixels, 3.0 us.
 __global__ __launch_bounds__(256) void qlinear_gap_kernel(const uint8_t* X, uint8_t* Y, int n, int hw, int c,
                                                           int x_zp, float m, int y_zp) {
-  const int ch = blockIdx.x * 256 + threadIdx.x;
+  __shared__ __align__(16) uint32_t part[4][64][4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ch = (blockIdx.x * 64 + lane) * 4, b = blockIdx.y;
+  const uint8_t* x = X + (size_t)b * hw * c + (ch < c ? ch : 0);
+  // bytes 0 and 2, 1 and 3 in 16-bit halves: 257 pixels before one overflows
+  uint32_t tot[4] = {0, 0, 0, 0};
+  for (int s0 = wave * kGapAhead; s0 < hw; s0 += 4 * kGapAhead) {
+    uint32_t v[kGapAhead], even = 0, odd = 0;
+#pragma unroll
+    for (int j = 0; j < kGapAhead; ++j)
+      v[j] = *reinterpret_cast<const uint32_t*>(x + (size_t)(s0 + j < hw ? s0 + j : hw - 1) * c);
+#pragma unroll
+    for (int j = 0; j < kGapAhead; ++j) {
+      const uint32_t w = s0 + j < hw ? v[j] : 0u;
+      even += w & 0x00ff00ffu;
+      odd += (w >> 8) & 0x00ff00ffu;
+    }
+    tot[0] += even & 0xffffu;
+    tot[1] += odd & 0xffffu;
+    tot[2] += even >> 16;
+    tot[3] += odd >> 16;
+  }
+  *reinterpret_cast<uint4*>(part[wave][lane]) = make_uint4(tot[0], tot[1], tot[2], tot[3]);
+  __syncthreads();
+  if (wave != 0 || ch >= c) return;
+  uint32_t out = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t sum = part[0][lane][j] + part[1][lane][j] + part[2][lane][j] + part[3][lane][j];
+    out |= (uint32_t)qgap_out((int)(sum - (uint32_t)hw * (uint32_t)x_zp), m, y_zp) << (8 * j);
+  }
+  *reinterpret_cast<uint32_t*>(Y + (size_t)b * c + ch) = out;
+}
+
+// The same for channel counts that are no multiple of 4: a byte a thread.
+__global__ __launch_bounds__(64) void qlinear_gap_byte_kernel(const uint8_t* X, uint8_t* Y, int n, int hw, int c,
+                                                              int x_zp, float m, int y_zp) {
+  const int ch = blockIdx.x * 64 + threadIdx.x;
   const int b = blockIdx.y;
   if (ch >= c || b >= n) return;
   const uint8_t* x = X + (size_t)b * hw * c + ch;
   int acc = 0;
+#pragma unroll 8
   for (int s = 0; s < hw; ++s) acc += (int)x[(size_t)s * c] - x_zp;
-  float q = rintf((float)acc * m) + (float)y_zp;
-  q = fminf(fmaxf(q, 0.0f), 255.0f);
-  Y[(size_t)b * c + ch] = (uint8_t)q;
+  Y[(size_t)b * c + ch] = qgap_out(acc, m, y_zp);
 }
 
 // dst[c][r] = src[r][c] for a rows x cols byte matrix (32 x 32 tiles through LDS).
@@ -305,11 +364,11 @@ void launch_gemm(hipStream_t st, int dtype, const void* a, const void* b, void* 
 }
 
 void launch_global_avg_pool(hipStream_t st, int dtype, const void* x, void* y, int n, int hw, int c) {
-  const dim3 g((unsigned)((c + 255) / 256), (unsigned)n);
+  const dim3 g((unsigned)(((long long)c + 63) / 64), (unsigned)n);
   if (dtype == F32)
-    hipLaunchKernelGGL((global_avg_pool_kernel<false>), g, dim3(256), 0, st, x, y, n, hw, c);
+    hipLaunchKernelGGL((global_avg_pool_kernel<false>), g, dim3(64), 0, st, x, y, n, hw, c);
   else if (dtype == F16)
-    hipLaunchKernelGGL((global_avg_pool_kernel<true>), g, dim3(256), 0, st, x, y, n, hw, c);
+    hipLaunchKernelGGL((global_avg_pool_kernel<true>), g, dim3(64), 0, st, x, y, n, hw, c);
   else
     fail(-2, "global average pool: dtype");
   DW_HIP(hipGetLastError());
@@ -341,8 +400,12 @@ namespace dw {
 
 void launch_qlinear_gap(hipStream_t st, const uint8_t* x, uint8_t* y, int n, int hw, int c, int x_zp, float m,
                         int y_zp) {
-  const dim3 g((unsigned)((c + 255) / 256), (unsigned)n);
-  hipLaunchKernelGGL(qlinear_gap_kernel, g, dim3(256), 0, st, x, y, n, hw, c, x_zp, m, y_zp);
+  if (c % 4 == 0)
+    hipLaunchKernelGGL(qlinear_gap_kernel, dim3((unsigned)((c + 255) / 256), (unsigned)n), dim3(256), 0, st, x, y, n, hw,
+                       c, x_zp, m, y_zp);
+  else
+    hipLaunchKernelGGL(qlinear_gap_byte_kernel, dim3((unsigned)((c + 63) / 64), (unsigned)n), dim3(64), 0, st, x, y, n,
+                       hw, c, x_zp, m, y_zp);
   DW_HIP(hipGetLastError());
 }
 
