@@ -26,10 +26,9 @@ namespace {
 
 // The multipliers of one launch's channels, passed by value: they live in
 // the caller's host array, and as kernel arguments they need no copy that
-// the host would have to wait for.  With the other arguments they stay below
-// the 4 KB an argument block holds.
-constexpr int kPrepChannels = 896;
-constexpr int kPackAhead = 3;  // k-steps a wave loads before it stores the first
+// the host would have to wait for.  With the other 64 bytes of arguments they
+// fill 4 KB.
+constexpr int kPrepChannels = 1008;
 struct PrepScales {
   float m[kPrepChannels];
 };
@@ -56,6 +55,7 @@ __device__ __forceinline__ void pack_weights_body(const uint8_t* __restrict__ w,
                                                   int cout, int cout_pad, int ksteps, const QconvPrep& q,
                                                   const float* m) {
   constexpr int RK = 4 / ESZ;  // rows of K in one output dword
+  constexpr int kPackAhead = Q ? 3 : 1;  // k-steps a wave loads before it stores the first
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int kg = lane & 15, quad = lane >> 4;
   const int cb = blockIdx.x * 16 + (Q ? q.c0 : 0);  // first channel of the workgroup
@@ -72,23 +72,30 @@ __device__ __forceinline__ void pack_weights_body(const uint8_t* __restrict__ w,
     }
   const int step = gridDim.y * waves;
   for (int s0 = blockIdx.y * waves + wave; s0 < ksteps; s0 += kPackAhead * step) {
+    // past K or c_out the last row or the first channels are read and
+    // replaced by zeros (a load under a condition would be a branch, waited
+    // for by itself)
     uint32_t r[kPackAhead][4];
 #pragma unroll
     for (int u = 0; u < kPackAhead; ++u) {
-      const int k0 = (s0 + u * step) * (64 / ESZ) + kg * RK;  // past K: zeros
-      if constexpr (ESZ == 1) {
+      const int k0 = (s0 + u * step) * (64 / ESZ) + kg * RK;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          r[u][j] = in && k0 + j < K ? *reinterpret_cast<const uint32_t*>(w + (size_t)(k0 + j) * cout + c) : 0u;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const uint2 v = in && k0 + j < K ? *reinterpret_cast<const uint2*>(w + ((size_t)(k0 + j) * cout + c) * 2)
-                                           : make_uint2(0u, 0u);
+      for (int j = 0; j < RK; ++j) {
+        const size_t at = (size_t)(k0 + j < K ? k0 + j : K - 1) * cout + (in ? c : 0);
+        if constexpr (ESZ == 1) {
+          r[u][j] = *reinterpret_cast<const uint32_t*>(w + at);
+        } else {
+          const uint2 v = *reinterpret_cast<const uint2*>(w + at * 2);
           r[u][2 * j] = v.x;
           r[u][2 * j + 1] = v.y;
         }
       }
+    }
+#pragma unroll
+    for (int u = 0; u < kPackAhead; ++u) {
+      const int k0 = (s0 + u * step) * (64 / ESZ) + kg * RK;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[u][j] = in && k0 + j * RK / 4 < K ? r[u][j] : 0u;
     }
 #pragma unroll
     for (int u = 0; u < kPackAhead; ++u) {
@@ -590,12 +597,15 @@ void launch_qconv_prep(hipStream_t st, const void* w_hwio, void* wpk, const int*
                        const float* m_host, int K, int cout, int cout_pad, int ksteps, int corr) {
   if (cout % 4 != 0 || cout_pad % 16 != 0) fail(-4, "qconv_prep: c_out must be a multiple of 4, its padding of 16");
   const dim3 block(64 * std::min(ksteps, 16));
-  for (int c0 = 0; c0 < cout_pad; c0 += kPrepChannels) {
-    PrepScales m{};
-    if (c0 < cout) memcpy(m.m, m_host + c0, sizeof(float) * std::min(kPrepChannels, cout - c0));
+  // a launch holds the multipliers of kPrepChannels channels; the last one
+  // also packs the padding channels, which have none
+  for (int c0 = 0; c0 < cout; c0 += kPrepChannels) {
+    PrepScales m;
+    memcpy(m.m, m_host + c0, sizeof(float) * std::min(kPrepChannels, cout - c0));
     const QconvPrep q{bias, bias_out, ms_out, corr, c0};
-    hipLaunchKernelGGL(qconv_prep_kernel, dim3(std::min(kPrepChannels, cout_pad - c0) / 16), block, 0, st,
-                       (const uint8_t*)w_hwio, (uint8_t*)wpk, K, cout, cout_pad, ksteps, q, m);
+    const int groups = (c0 + kPrepChannels < cout ? kPrepChannels : cout_pad - c0) / 16;
+    hipLaunchKernelGGL(qconv_prep_kernel, dim3(groups), block, 0, st, (const uint8_t*)w_hwio, (uint8_t*)wpk, K, cout,
+                       cout_pad, ksteps, q, m);
   }
   DW_HIP(hipGetLastError());
 }
