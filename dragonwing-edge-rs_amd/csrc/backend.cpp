@@ -11,6 +11,8 @@
 
 #include <algorithm>
 #include <exception>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/dw_hip.h"
@@ -50,9 +52,93 @@ void Backend::upload_async(void* dst, const void* src, size_t bytes) {
   DW_HIP(hipStreamSynchronize(stream));
 }
 
+// Chunks `thread`, thread + threads, ... of a download: the copy of one chunk
+// out of its page-locked slot runs while the device fills the thread's other
+// slot.  Every copy that was queued has ended when this returns.
+hipError_t Backend::copy_chunks(uint8_t* dst, const uint8_t* src, size_t bytes, size_t chunk, int thread,
+                                int threads) {
+  hipError_t err = hipSetDevice(device);
+  const size_t n = (bytes + chunk - 1) / chunk;
+  auto queue = [&](size_t c, int slot) -> hipError_t {
+    const size_t len = std::min(chunk, bytes - c * chunk);
+    hipError_t e = hipMemcpyAsync(slots + (size_t)slot * kSlotBytes, src + c * chunk, len, hipMemcpyDeviceToHost,
+                                  stream);
+    return e == hipSuccess ? hipEventRecord(slot_ev[slot], stream) : e;
+  };
+  size_t next = (size_t)thread, done = next;  // the next chunk to queue, to copy out
+  int in = 0, out = 0;                        // their places among the thread's two slots
+  const int first = 2 * thread;
+  while (err == hipSuccess && done < n) {
+    while (err == hipSuccess && next < n && next <= done + (size_t)threads) {
+      err = queue(next, first + in);
+      next += (size_t)threads;
+      in ^= 1;
+    }
+    if (err == hipSuccess) err = hipEventSynchronize(slot_ev[first + out]);
+    if (err == hipSuccess)
+      memcpy(dst + done * chunk, slots + (size_t)(first + out) * kSlotBytes, std::min(chunk, bytes - done * chunk));
+    done += (size_t)threads;
+    out ^= 1;
+  }
+  if (err != hipSuccess) (void)hipStreamSynchronize(stream);
+  return err;
+}
+
+// Through the page-locked slots: the driver's own copy to ordinary memory
+// runs at 18 GB/s, and one to page-locked memory at 56 GB/s of which a thread
+// moves 31 GB/s on (less into pages touched for the first time), so from 4 MiB
+// on four threads copy.  Measured into warm memory: 0.46 MB 37 us, 1.8 MB 90
+// us, 59 MB 1.56 ms (38 GB/s).
+void Backend::download(void* dst, const void* src, size_t bytes) {
+  hipPointerAttribute_t at{};
+  if (bytes && hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered) {
+    // memory the runtime knows (page-locked by the caller): the device copies there directly
+    DW_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
+  } else if (bytes) {
+    (void)hipGetLastError();  // of an address that the runtime does not know
+    if (!slots) {
+      for (auto& e : slot_ev)
+        if (!e) DW_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      DW_HIP(hipHostMalloc((void**)&slots, kSlots * kSlotBytes, hipHostMallocDefault));
+    }
+    uint8_t* d = (uint8_t*)dst;
+    const uint8_t* s = (const uint8_t*)src;
+    // a chunk costs about 10 us beside its bytes, which half a MiB hides; large
+    // downloads take whole slots
+    const size_t mib = (size_t)1 << 20;
+    const size_t chunk = bytes >= 16 * mib ? kSlotBytes
+                         : bytes <= mib    ? bytes
+                                           : std::min(mib, (bytes / 2 + 4095) & ~(size_t)4095);
+    hipError_t err[kCopyThreads] = {};
+    if (bytes >= 4 * mib) {
+      std::thread helper[kCopyThreads];
+      for (int t = 1; t < kCopyThreads; ++t) try {
+          helper[t] = std::thread([=, &err] { err[t] = copy_chunks(d, s, bytes, chunk, t, kCopyThreads); });
+        } catch (const std::system_error&) {
+          // no thread to be had: its share is copied below
+        }
+      err[0] = copy_chunks(d, s, bytes, chunk, 0, kCopyThreads);
+      for (int t = 1; t < kCopyThreads; ++t) {
+        if (helper[t].joinable())
+          helper[t].join();
+        else
+          err[t] = copy_chunks(d, s, bytes, chunk, t, kCopyThreads);
+      }
+    } else {
+      err[0] = copy_chunks(d, s, bytes, chunk, 0, 1);
+    }
+    for (hipError_t e : err) hip_check(e, "download");
+    return;
+  }
+  DW_HIP(hipStreamSynchronize(stream));
+}
+
 Backend::~Backend() {
   if (stream) {
     (void)hipStreamSynchronize(stream);
+    if (slots) (void)hipHostFree(slots);
+    for (auto& e : slot_ev)
+      if (e) (void)hipEventDestroy(e);
     for (auto& w : ws)
       if (w.ptr) (void)hipFree(w.ptr);
     (void)hipStreamDestroy(stream);
@@ -271,11 +357,7 @@ int dw_hip_download(dw_hip_backend* be, const dw_hip_buffer* src, void* dst, siz
   if (len != src->len)
     dw::fail(DW_ERR_INVALID, "download size mismatch: buffer " + std::to_string(src->len) +
                                  " bytes, destination " + std::to_string(len) + " bytes");
-  DW_HIP(hipStreamSynchronize(b->stream));
-  if (len) {
-    DW_HIP(hipMemcpyAsync(dst, src->ptr, len, hipMemcpyDeviceToHost, b->stream));
-    DW_HIP(hipStreamSynchronize(b->stream));
-  }
+  b->download(dst, src->ptr, len);
   API_END
 }
 

@@ -62,7 +62,19 @@ struct Backend {
 
   void* workspace(int slot, size_t bytes);
   void upload_async(void* dst, const void* src, size_t bytes);
+  // The stream's work so far, then `bytes` from the device to `dst` (any host
+  // memory), complete on return.  Call with mu held.
+  void download(void* dst, const void* src, size_t bytes);
   ~Backend();
+
+ private:
+  // Page-locked slots that downloads go through, two for each copying thread
+  // (made by the first download, freed with the backend).
+  static constexpr int kCopyThreads = 4, kSlots = 2 * kCopyThreads;
+  static constexpr size_t kSlotBytes = (size_t)2 << 20;
+  uint8_t* slots = nullptr;
+  hipEvent_t slot_ev[kSlots] = {};
+  hipError_t copy_chunks(uint8_t* dst, const uint8_t* src, size_t bytes, size_t chunk, int thread, int threads);
 };
 
 inline void hold(Backend* b) { b->holds.fetch_add(1, std::memory_order_relaxed); }

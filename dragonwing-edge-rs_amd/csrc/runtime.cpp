@@ -3164,27 +3164,38 @@ int dw_hip_graph_tensor_shape(dw_hip_graph_runtime* rth, const char* name, int64
   API_END
 }
 
-static void download_tensor(dw::Runtime& rt, const std::string& name, std::vector<uint8_t>& out) {
-  dw::RtTensor& t = rt.T(name);
-  if (!t.base) dw::fail(DW_ERR_RUNTIME, "tensor " + name + " is not materialized");
-  DW_HIP(hipStreamSynchronize(rt.be->stream));
+// A tensor's dense bytes at `dst` (host), complete on return.  A channel
+// slice is gathered on the device first: a strided copy to the host goes row
+// by row (55 ms for one 640x640 image's three head outputs, 2.4 MB).
+static void download_tensor(dw::Runtime& rt, const dw::RtTensor& t, void* dst) {
   const size_t es = dw::dtype_size(t.dtype);
-  out.resize(t.bytes());
-  DW_HIP(hipMemcpy2D(out.data(), t.c * es, (const uint8_t*)t.base + (size_t)t.abs_off * es,
-                     (size_t)t.pix_stride * es, t.c * es, (size_t)t.pixels(), hipMemcpyDeviceToHost));
+  hipStream_t st = rt.be->stream;
+  const uint8_t* src = (const uint8_t*)t.base + (size_t)t.abs_off * es;
+  if (t.pix_stride != t.c && t.pixels() > 1) {
+    void* dense = rt.be->workspace(dw::Backend::WS_POST, t.bytes());
+    dw::launch_copy_channels(st, t.view(), {dense, (int)t.c, 0}, (int)t.pixels(), (int)t.c, (int)es);
+    src = (const uint8_t*)dense;
+  }
+  rt.be->download(dst, src, t.bytes());
+}
+
+static const dw::RtTensor& output_tensor(dw::Runtime& rt, const char* name) {
+  if (!name) dw::fail(DW_ERR_INVALID, "null name");
+  const dw::RtTensor& t = rt.T(name);
+  if (!t.base) dw::fail(DW_ERR_RUNTIME, std::string("tensor ") + name + " is not materialized");
+  return t;
 }
 
 int dw_hip_graph_get_output_bytes(dw_hip_graph_runtime* rth, const char* name, void* data, size_t len) {
   API_BEGIN
   dw::Runtime& rt = R(rth);
   std::lock_guard<std::mutex> lock(rt.be->mu);
-  if (!name) dw::fail(DW_ERR_INVALID, "null name");
-  std::vector<uint8_t> buf;
-  download_tensor(rt, name, buf);
-  if (len != buf.size())
-    dw::fail(DW_ERR_RUNTIME, "output size mismatch: expected " + std::to_string(buf.size()) + ", got " +
+  const dw::RtTensor& t = output_tensor(rt, name);
+  if (len != t.bytes())
+    dw::fail(DW_ERR_RUNTIME, "output size mismatch: expected " + std::to_string(t.bytes()) + ", got " +
                                  std::to_string(len));
-  memcpy(data, buf.data(), len);
+  if (len && !data) dw::fail(DW_ERR_INVALID, "null data");
+  download_tensor(rt, t, data);
   API_END
 }
 
@@ -3192,21 +3203,22 @@ int dw_hip_graph_get_output_f32(dw_hip_graph_runtime* rth, const char* name, flo
   API_BEGIN
   dw::Runtime& rt = R(rth);
   std::lock_guard<std::mutex> lock(rt.be->mu);
-  if (!name) dw::fail(DW_ERR_INVALID, "null name");
-  dw::RtTensor& t = rt.T(name);
-  std::vector<uint8_t> buf;
-  download_tensor(rt, name, buf);
+  const dw::RtTensor& t = output_tensor(rt, name);
   const size_t n = (size_t)(t.pixels() * t.c);
   if (count != n) dw::fail(DW_ERR_RUNTIME, "output size mismatch");
+  if (t.dtype != dw::F32 && t.dtype != dw::F16 && t.dtype != dw::U8)
+    dw::fail(DW_ERR_RUNTIME, "unsupported dtype for get_output_f32");
   if (t.dtype == dw::F32) {
-    memcpy(data, buf.data(), n * 4);
-  } else if (t.dtype == dw::F16) {
+    download_tensor(rt, t, data);
+    return DW_OK;
+  }
+  std::vector<uint8_t> buf(t.bytes());
+  download_tensor(rt, t, buf.data());
+  if (t.dtype == dw::F16) {
     const uint16_t* h = (const uint16_t*)buf.data();
     for (size_t i = 0; i < n; ++i) data[i] = f16_to_f32_ref(h[i]);
   } else if (t.dtype == dw::U8) {
     for (size_t i = 0; i < n; ++i) data[i] = (float)((int)buf[i] - t.zp) * t.scale;
-  } else {
-    dw::fail(DW_ERR_RUNTIME, "unsupported dtype for get_output_f32");
   }
   API_END
 }
