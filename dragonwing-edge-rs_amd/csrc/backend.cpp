@@ -6,6 +6,7 @@
 #include "backend.h"
 
 #include <math.h>
+#include <stddef.h>
 #include <stdint.h>
 #include <string.h>
 
@@ -1079,9 +1080,11 @@ int dw_hip_yolo_postprocess(dw_hip_backend* be, const dw_hip_buffer* raw, size_t
   // workspace: keys, per-anchor detections, then per image nmax-sized arrays
   const size_t A = num_det;
   auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  // the results (counts, then the kept detections of all images packed) lie
+  // together at the end
   const size_t o_keys = 0, o_det = o_keys + al(n * A * 8), o_sa = o_det + al(n * A * 24);
-  const size_t o_pp = o_sa + al(n * nmax * 4), o_od = o_pp + al(n * nmax * 4);
-  const size_t o_op = o_od + al(n * nmax * 24), o_cnt = o_op + al(n * nmax * 4), total = o_cnt + al(n * 16);
+  const size_t o_pp = o_sa + al(n * nmax * 4), o_cur = o_pp + al(n * nmax * 4), o_cnt = o_cur + 256;
+  const size_t o_kept = o_cnt + n * 16, total = o_kept + n * nmax * sizeof(dw::DwKept);
   uint8_t* ws = (uint8_t*)bk->workspace(Backend::WS_POST, total);
   dw::PostprocessArgs a{};
   a.raw = (const float*)raw->ptr;
@@ -1101,30 +1104,31 @@ int dw_hip_yolo_postprocess(dw_hip_backend* be, const dw_hip_buffer* raw, size_t
   a.det = (dw::DwDetection*)(ws + o_det);
   a.sorted_anchor = (int*)(ws + o_sa);
   a.part_pos = (int*)(ws + o_pp);
-  a.out_det = (dw::DwDetection*)(ws + o_od);
-  a.out_pos = (int*)(ws + o_op);
+  a.cursor = (int*)(ws + o_cur);
   a.counts = (int*)(ws + o_cnt);
+  a.kept = (dw::DwKept*)(ws + o_kept);
   dw::launch_yolo_postprocess(bk->stream, a);
-  std::vector<int> cnt(n * 4);
-  DW_HIP(hipMemcpyAsync(cnt.data(), a.counts, n * 16, hipMemcpyDeviceToHost, bk->stream));
-  DW_HIP(hipStreamSynchronize(bk->stream));
-  size_t maxk = 0;
+  // one download takes the counts and as many kept detections as frames
+  // usually have; a second one the rest
+  const size_t guess = n * (16 + 512 * sizeof(dw::DwKept)), most = total - o_cnt;
+  std::vector<uint8_t> res(std::min(guess, most));
+  bk->download(res.data(), ws + o_cnt, res.size());
+  const int* cnt = (const int*)res.data();
+  size_t kept = 0;
   for (size_t b = 0; b < n; ++b) {
     if (cnt[4 * b + 2])
       dw::fail(DW_ERR_UNSUPPORTED, "postprocess: image " + std::to_string(b) + " has " +
                                        std::to_string(cnt[4 * b]) + " candidates over the threshold (at most " +
                                        std::to_string(nmax) + ")");
-    maxk = std::max(maxk, (size_t)cnt[4 * b + 1]);
+    kept += (size_t)cnt[4 * b + 1];
   }
-  std::vector<dw::DwDetection> kd(n * (size_t)nmax);
-  std::vector<int> kp(n * (size_t)nmax);
-  if (maxk) {
-    DW_HIP(hipMemcpy2DAsync(kd.data(), (size_t)nmax * 24, a.out_det, (size_t)nmax * 24, maxk * 24, n,
-                            hipMemcpyDeviceToHost, bk->stream));
-    DW_HIP(hipMemcpy2DAsync(kp.data(), (size_t)nmax * 4, a.out_pos, (size_t)nmax * 4, maxk * 4, n,
-                            hipMemcpyDeviceToHost, bk->stream));
-    DW_HIP(hipStreamSynchronize(bk->stream));
+  const size_t have = res.size(), need_bytes = n * 16 + kept * sizeof(dw::DwKept);
+  if (need_bytes > have) {
+    res.resize(need_bytes);
+    cnt = (const int*)res.data();
+    bk->download(res.data() + have, ws + o_cnt + have, need_bytes - have);
   }
+  const uint8_t* kd = res.data() + n * 16;
   // The reference removes suppressed entries from the back with swap_remove
   // (postprocess.rs:235-242): walking the sorted positions downwards, a
   // suppressed slot takes the current last element and the list shrinks.
@@ -1138,8 +1142,14 @@ int dw_hip_yolo_postprocess(dw_hip_backend* be, const dw_hip_buffer* raw, size_t
       over = true;
       continue;
     }
+    const uint8_t* mine = kd + (size_t)cnt[4 * b + 3] * sizeof(dw::DwKept);
+    auto entry = [&](int i) { return mine + (size_t)i * sizeof(dw::DwKept); };
     slot.assign((size_t)nc_b, -1);
-    for (int i = 0; i < k; ++i) slot[(size_t)kp[b * nmax + i]] = i;
+    for (int i = 0; i < k; ++i) {
+      int pos;
+      memcpy(&pos, entry(i) + offsetof(dw::DwKept, pos), sizeof pos);
+      slot[(size_t)pos] = i;
+    }
     int len = nc_b;
     for (int i = nc_b - 1; i >= 0; --i)
       if (slot[(size_t)i] < 0) {
@@ -1147,7 +1157,7 @@ int dw_hip_yolo_postprocess(dw_hip_backend* be, const dw_hip_buffer* raw, size_t
         --len;
       }
     dw_detection* o = out + b * cap;
-    for (int i = 0; i < len; ++i) memcpy(&o[i], &kd[b * nmax + (size_t)slot[(size_t)i]], sizeof(dw_detection));
+    for (int i = 0; i < len; ++i) memcpy(&o[i], entry(slot[(size_t)i]), sizeof(dw_detection));
   }
   if (over) dw::fail(DW_ERR_INVALID, "postprocess: more detections than cap in an image (see counts)");
   API_END

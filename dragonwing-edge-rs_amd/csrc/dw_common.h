@@ -340,6 +340,12 @@ struct DwDetection {
   uint32_t class_id;
   float confidence;
 };
+// A detection that NMS kept and its place among its image's candidates in
+// sorted order.
+struct DwKept {
+  DwDetection det;
+  int pos;
+};
 // Per-level NHWC head outputs [n][h][w][pix], 4 * reg_max box channels
 // then nc class channels at the start of each pixel.
 struct DetectTailArgs {
@@ -361,9 +367,9 @@ struct PostprocessArgs {
   DwDetection* det;
   int* sorted_anchor;
   int* part_pos;
-  DwDetection* out_det;
-  int* out_pos;
-  int* counts;
+  DwKept* kept;  // n * nmax entries: the images' kept detections, packed
+  int* counts;   // [n][4]: candidates, kept, overflow, first entry in `kept`
+  int* cursor;   // one int
 };
 size_t pp_nms_lds_bytes(int nmax);
 void launch_yolo_postprocess(hipStream_t st, const PostprocessArgs& a);

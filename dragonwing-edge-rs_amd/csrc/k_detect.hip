@@ -15,8 +15,9 @@
 //   pp_candidates_kernel  decode_detections_v8 (:78-146) for every anchor:
 //                         best class, threshold, corners, clamp; a 64-bit
 //                         sort key (confidence descending, anchor ascending);
-//   pp_nms_kernel         one workgroup per image: bitonic sort of the keys
-//                         in LDS (the reference's stable sort by confidence),
+//   pp_nms_kernel         one workgroup per image: the keys over the threshold
+//                         gathered and bitonically sorted in registers or LDS
+//                         (the reference's stable sort by confidence),
 //                         a stable partition by class, greedy NMS per class
 //                         on LDS-resident boxes, one wave per class
 //                         (nms, :214-243; nms_agnostic as one class), and the
@@ -34,8 +35,9 @@ namespace {
 struct TailLevels {
   const void* x[4];
   int h[4], w[4];
-  int start[4];
-  int pix[4];  // elements per pixel
+  int start[4];  // first anchor of the level
+  int tile0[4];  // first 64-anchor tile of the level
+  int pix[4];    // elements per pixel
   float stride[4];
   int levels;
   int A;
@@ -49,6 +51,127 @@ __device__ __forceinline__ float tail_ld(const void* p, size_t i) {
     return ((const float*)p)[i];
 }
 
+// One side's DFL from its logits ld(0..reg_max-1): softmax, then the
+// expectation's fma chain.  R > 0: reg_max as a constant, so that the
+// exponentials stay in registers; 0: any reg_max, each computed twice.
+template <int R, typename Ld>
+__device__ __forceinline__ float dfl_side(int reg_max, Ld ld) {
+  float mx = -INFINITY, sum = 0.0f, acc = 0.0f;
+  if constexpr (R > 0) {
+    float e[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      e[k] = ld(k);
+      mx = fmaxf(mx, e[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      e[k] = expf(e[k] - mx);
+      sum += e[k];
+    }
+    const float inv = __fdiv_rn(1.0f, sum);
+#pragma unroll
+    for (int k = 0; k < R; ++k) acc = fmaf(e[k] * inv, (float)k, acc);
+  } else {
+    for (int k = 0; k < reg_max; ++k) mx = fmaxf(mx, ld(k));
+    for (int k = 0; k < reg_max; ++k) sum += expf(ld(k) - mx);
+    const float inv = __fdiv_rn(1.0f, sum);
+    for (int k = 0; k < reg_max; ++k) acc = fmaf(expf(ld(k) - mx) * inv, (float)k, acc);
+  }
+  return acc;
+}
+
+// Row j of the box (centre x, centre y, width, height) of the anchor at grid
+// cell (gx, gy), from its four distances.
+__device__ __forceinline__ float box_row(int j, const float d[4], int gx, int gy, float st) {
+  const float ax = (float)gx + 0.5f, ay = (float)gy + 0.5f;
+  const float lo = j & 1 ? ay - d[1] : ax - d[0];
+  const float hi = j & 1 ? ay + d[3] : ax + d[2];
+  return (j < 2 ? __fdiv_rn(lo + hi, 2.0f) : hi - lo) * st;
+}
+__device__ __forceinline__ float sigmoid_rn(float v) { return __fdiv_rn(1.0f, 1.0f + expf(-v)); }
+
+// A workgroup takes 64 consecutive anchors of one level and image: their
+// pixels, 288 contiguous bytes each for an f16 head of 144 channels, are read
+// as whole lines (every load of a thread in flight together), widened once
+// and kept in LDS as f32 with an odd row stride, so that 64 lanes at one
+// channel of 64 anchors fall on different banks.  A wave owns one box side
+// (its DFL, then one box row) and a quarter of the classes; every output row
+// is written as 64 consecutive floats.  Bound by exp and the divisions once
+// the bytes stream (624 B an anchor): eight 640x640 images (42 MB) take
+// 22 us, against 83 us for a thread per anchor reading its own pixel two
+// bytes at a time.
+constexpr int kTailAnchors = 64;
+// dwords a thread may hold: 192 f16 or 160 f32 channels
+__host__ __device__ constexpr int tail_loads(bool h) { return h ? 24 : 40; }
+template <bool H, int R>
+__global__ __launch_bounds__(256) void detect_tail_tile_kernel(TailLevels L, float* out, int nc, int reg_max) {
+  extern __shared__ float tile[];  // [64][ld], then the distances [4][64]
+  const int chans = 4 * reg_max + nc, ld = chans | 1;
+  float* dist = tile + kTailAnchors * ld;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, b = blockIdx.y;
+  int s = 0;
+  while (s + 1 < L.levels && (int)blockIdx.x >= L.tile0[s + 1]) ++s;
+  const int hw = L.h[s] * L.w[s];
+  const int a0 = ((int)blockIdx.x - L.tile0[s]) * kTailAnchors;  // first anchor in the level
+  const int live = min(kTailAnchors, hw - a0);
+  // dword i of the tile: anchor i / dw, its dword i % dw; 256 dwords further
+  // on is (256 / dw, 256 % dw) further on
+  const int dw = H ? chans / 2 : chans, pixdw = H ? L.pix[s] / 2 : L.pix[s];
+  const uint32_t* x = (const uint32_t*)L.x[s] + ((size_t)b * hw + a0) * (size_t)pixdw;
+  const int sa = 256 / dw, sr = 256 % dw;
+  {
+    constexpr int kTailLoads = tail_loads(H);
+    uint32_t v[kTailLoads];
+    int a = t / dw, r = t % dw;
+#pragma unroll
+    for (int i = 0; i < kTailLoads; ++i) {
+      v[i] = x[a < live ? (size_t)a * pixdw + r : 0];
+      a += sa;
+      r += sr;
+      if (r >= dw) {
+        r -= dw;
+        ++a;
+      }
+    }
+    a = t / dw;
+    r = t % dw;
+#pragma unroll
+    for (int i = 0; i < kTailLoads; ++i) {
+      if (a < live) {
+        if constexpr (H) {
+          tile[a * ld + 2 * r] = h2f((uint16_t)v[i]);
+          tile[a * ld + 2 * r + 1] = h2f((uint16_t)(v[i] >> 16));
+        } else {
+          tile[a * ld + r] = __builtin_bit_cast(float, v[i]);
+        }
+      }
+      a += sa;
+      r += sr;
+      if (r >= dw) {
+        r -= dw;
+        ++a;
+      }
+    }
+  }
+  __syncthreads();
+  const float* row = tile + min(lane, live - 1) * ld;  // idle lanes repeat the last anchor
+  dist[wave * 64 + lane] = dfl_side<R>(reg_max, [&](int k) { return row[wave * reg_max + k]; });
+  const size_t A = (size_t)L.A;
+  float* o = out + (size_t)b * (4 + nc) * A + L.start[s] + a0 + lane;
+  for (int c = wave; c < nc; c += 4) {
+    const float v = sigmoid_rn(row[4 * reg_max + c]);
+    if (lane < live) o[(size_t)(4 + c) * A] = v;
+  }
+  __syncthreads();
+  const float d[4] = {dist[lane], dist[64 + lane], dist[128 + lane], dist[192 + lane]};
+  const int gy = (a0 + lane) / L.w[s], gx = (a0 + lane) - gy * L.w[s];
+  const float v = box_row(wave, d, gx, gy, L.stride[s]);
+  if (lane < live) o[(size_t)wave * A] = v;
+}
+
+// Any head (channels that do not pair into dwords, or more than a thread of
+// the tile kernel holds): a thread per anchor, straight from memory.
 template <bool H>
 __global__ __launch_bounds__(256) void detect_tail_kernel(TailLevels L, float* out, int nc, int reg_max) {
   const int a = blockIdx.x * 256 + threadIdx.x;
@@ -61,35 +184,13 @@ __global__ __launch_bounds__(256) void detect_tail_kernel(TailLevels L, float* o
   const int gx = local - gy * L.w[s];
   const size_t px = (((size_t)b * L.h[s] + gy) * L.w[s] + gx) * (size_t)L.pix[s];
   const void* x = L.x[s];
-  float* o = out + (size_t)b * (4 + nc) * L.A + a;
-  float d[4];
-  for (int j = 0; j < 4; ++j) {
-    const size_t base = px + (size_t)j * reg_max;
-    float mx = -INFINITY;
-    for (int k = 0; k < reg_max; ++k) mx = fmaxf(mx, tail_ld<H>(x, base + k));
-    float sum = 0.0f;
-    for (int k = 0; k < reg_max; ++k) sum += expf(tail_ld<H>(x, base + k) - mx);
-    const float inv = __fdiv_rn(1.0f, sum);
-    float acc = 0.0f;
-    for (int k = 0; k < reg_max; ++k) {
-      const float p = expf(tail_ld<H>(x, base + k) - mx) * inv;
-      acc = fmaf(p, (float)k, acc);
-    }
-    d[j] = acc;
-  }
-  const float ax = (float)gx + 0.5f, ay = (float)gy + 0.5f;
-  const float x1 = ax - d[0], y1 = ay - d[1], x2 = ax + d[2], y2 = ay + d[3];
-  const float st = L.stride[s];
   const size_t A = (size_t)L.A;
-  o[0] = __fdiv_rn(x1 + x2, 2.0f) * st;
-  o[A] = __fdiv_rn(y1 + y2, 2.0f) * st;
-  o[2 * A] = (x2 - x1) * st;
-  o[3 * A] = (y2 - y1) * st;
-  const size_t cbase = px + (size_t)4 * reg_max;
-  for (int c = 0; c < nc; ++c) {
-    const float v = tail_ld<H>(x, cbase + c);
-    o[(size_t)(4 + c) * A] = __fdiv_rn(1.0f, 1.0f + expf(-v));
-  }
+  float* o = out + (size_t)b * (4 + nc) * A + a;
+  float d[4];
+  for (int j = 0; j < 4; ++j)
+    d[j] = dfl_side<0>(reg_max, [&](int k) { return tail_ld<H>(x, px + (size_t)j * reg_max + k); });
+  for (int j = 0; j < 4; ++j) o[(size_t)j * A] = box_row(j, d, gx, gy, L.stride[s]);
+  for (int c = 0; c < nc; ++c) o[(size_t)(4 + c) * A] = sigmoid_rn(tail_ld<H>(x, px + (size_t)4 * reg_max + c));
 }
 
 // ---------------------------------------------------------------------------
@@ -101,14 +202,13 @@ struct PPArgs {
   float sx, sy, img_w, img_h, conf, iou;
   int agnostic;
   int nmax;          // capacity of the per-image arrays below
-  int sort_n;        // power of two >= A
   unsigned long long* keys;  // [n][A]
   DwDetection* det;          // [n][A], per anchor
   int* sorted_anchor;        // [n][nmax]
   int* part_pos;             // [n][nmax]
-  DwDetection* out_det;      // [n][nmax]
-  int* out_pos;              // [n][nmax]
-  int* counts;               // [n][4]: candidates, kept, overflow
+  DwKept* kept;              // every image's kept detections, one image after another
+  int* counts;               // [n][4]: candidates, kept, overflow, first of the image's in `kept`
+  int* cursor;               // entries of `kept` taken
 };
 
 __global__ __launch_bounds__(256) void pp_candidates_kernel(PPArgs p) {
@@ -118,15 +218,22 @@ __global__ __launch_bounds__(256) void pp_candidates_kernel(PPArgs p) {
   const size_t A = (size_t)p.A;
   const float* r = p.raw + (size_t)b * (4 + p.nc) * A + a;
   const float cx = r[0], cy = r[A], w = r[2 * A], h = r[3 * A];
+  // the class rows 16 at a time, so that their loads are in flight together
+  // (past the last class its value again, which is not greater)
   int best = 0;
   float best_conf = 0.0f;
-  for (int c = 0; c < p.nc; ++c) {
-    const float v = r[(size_t)(4 + c) * A];
-    if (v > best_conf) {
-      best_conf = v;
-      best = c;
-    }
+  for (int c0 = 0; c0 < p.nc; c0 += 16) {
+    float v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) v[j] = r[(size_t)(4 + min(c0 + j, p.nc - 1)) * A];
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      if (v[j] > best_conf) {
+        best_conf = v[j];
+        best = c0 + j;
+      }
   }
+  if (a == 0 && b == 0) *p.cursor = 0;  // for pp_nms_kernel, which follows
   unsigned long long key = ~0ull;
   if (!(best_conf < p.conf)) {
     const float hw = __fdiv_rn(w, 2.0f), hh = __fdiv_rn(h, 2.0f);
@@ -167,19 +274,39 @@ constexpr int kNmsThreads = 1024;
 constexpr int kNmsPer = (kPPMaxCandidates + kNmsThreads - 1) / kNmsThreads;
 
 // LDS layout (bytes), phase by phase:
-//   [0, 16 nmax)            sort keys (sort_n * 8 <= 16 nmax), then class ids
+//   [0, 16 nmax)            sort keys (at most 16384 of 8 bytes), then class ids
 //                           of the sorted candidates (u16), then the boxes in
 //                           class-partitioned order (float4)
 //   [16 nmax, 17 nmax)      keep flags (partitioned order)
 //   then 1024 ints          per-class counts / scan scratch
 //   then 1024 ints          per-class offsets
 //   then nmax / 32 words    kept bitmap over sorted positions
-//   then 4 ints             candidate count, next class
+//   then 4 ints             candidate count, next class, first kept entry
 __host__ __device__ constexpr size_t nms_lds_bytes(int nmax) {
   return (size_t)17 * nmax + 2 * 1024 * 4 + (size_t)((nmax + 31) / 32) * 4 + 16;
 }
 
+// Inclusive scan over the workgroup's threads (wsum: an int per wave).
+__device__ __forceinline__ int block_scan(int v, int* wsum) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int add = __shfl_up(v, d);
+    v += lane >= d ? add : 0;
+  }
+  __syncthreads();  // an earlier scan's reads are done
+  if (lane == 63) wsum[wave] = v;
+  __syncthreads();
+  for (int w = 0; w < kNmsThreads / 64 - 1; ++w) v += w < wave ? wsum[w] : 0;
+  return v;
+}
+
+// One workgroup per image, a chain of short phases between barriers, so its
+// time is their latencies: sorting only the candidates (a few hundred, in
+// registers) and scanning through lane shuffles, eight 640x640 frames of
+// about 350 candidates take 31 us, against 243 us with a sort of 16384 keys.
 __global__ __launch_bounds__(kNmsThreads) void pp_nms_kernel(PPArgs p) {
+  __shared__ int wsum[kNmsThreads / 64];
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int nmax = p.nmax;
   unsigned long long* sk = (unsigned long long*)smem;
@@ -192,40 +319,86 @@ __global__ __launch_bounds__(kNmsThreads) void pp_nms_kernel(PPArgs p) {
   int* sn = (int*)(kbits + (nmax + 31) / 32);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int b = blockIdx.x;
-  const int A = p.A, S = p.sort_n;
+  const int A = p.A;
   const int ncls = p.agnostic ? 1 : p.nc;
 
   if (tid == 0) {
     sn[0] = 0;
     sn[1] = 0;
   }
-  for (int i = tid; i < S; i += kNmsThreads) sk[i] = i < A ? p.keys[(size_t)b * A + i] : ~0ull;
   __syncthreads();
-  // bitonic sort, ascending: confidence descending, then anchor ascending
-  for (int k = 2; k <= S; k <<= 1)
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = tid; i < S; i += kNmsThreads) {
-        const int ixj = i ^ j;
-        if (ixj > i) {
-          const unsigned long long u = sk[i], v = sk[ixj];
-          if ((u > v) == ((i & k) == 0)) {
-            sk[i] = v;
-            sk[ixj] = u;
-          }
-        }
+  // The keys over the threshold, gathered in any order (they are distinct,
+  // so the sort decides): a few hundred of 8400 on an ordinary frame.
+  // All loads first: at most 16384 anchors, 16 a thread.
+  {
+    unsigned long long key[16384 / kNmsThreads];
+#pragma unroll
+    for (int u = 0; u < 16384 / kNmsThreads; ++u)
+      key[u] = p.keys[(size_t)b * A + min(u * kNmsThreads + tid, A - 1)];
+#pragma unroll
+    for (int u = 0; u < 16384 / kNmsThreads; ++u) {
+      const bool in = u * kNmsThreads + tid < A && key[u] != ~0ull;
+      const unsigned long long m = __ballot(in);
+      if (m) {
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&sn[0], __popcll(m));
+        at = __shfl(at, 0);
+        if (in) sk[at + __popcll(m & ((1ull << lane) - 1))] = key[u];
       }
-      __syncthreads();
     }
-  for (int i = tid; i < S; i += kNmsThreads)
-    if (sk[i] != ~0ull && (i + 1 == S || sk[i + 1] == ~0ull)) sn[0] = i + 1;
+  }
   __syncthreads();
   const int n = sn[0];
+  // bitonic sort, ascending: confidence descending, then anchor ascending
+  int S = 64;
+  while (S < n) S <<= 1;
+  if (S <= kNmsThreads) {
+    // a key per thread: partners in the same wave trade through lane
+    // shuffles, only the others through LDS and barriers (6 of 45 steps at 512)
+    unsigned long long key = tid < n ? sk[tid] : ~0ull;
+    __syncthreads();
+    for (int k = 2; k <= S; k <<= 1)
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        unsigned long long other;
+        if (j >= 64) {
+          sk[tid] = key;
+          __syncthreads();
+          other = sk[tid ^ j];
+          __syncthreads();
+        } else {
+          other = __shfl_xor(key, j);
+        }
+        // the lower place of an ascending pair keeps the smaller key
+        const bool low = ((tid & j) == 0) == ((tid & k) == 0);
+        key = (key < other) == low ? key : other;
+      }
+    sk[tid] = key;
+    __syncthreads();
+  } else {
+    for (int i = n + tid; i < S; i += kNmsThreads) sk[i] = ~0ull;
+    __syncthreads();
+    for (int k = 2; k <= S; k <<= 1)
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        for (int i = tid; i < S; i += kNmsThreads) {
+          const int ixj = i ^ j;
+          if (ixj > i) {
+            const unsigned long long u = sk[i], v = sk[ixj];
+            if ((u > v) == ((i & k) == 0)) {
+              sk[i] = v;
+              sk[ixj] = u;
+            }
+          }
+        }
+        __syncthreads();
+      }
+  }
   int* cnt = p.counts + 4 * b;
   if (n > nmax) {
     if (tid == 0) {
       cnt[0] = n;
       cnt[1] = 0;
       cnt[2] = 1;
+      cnt[3] = 0;
     }
     return;
   }
@@ -253,17 +426,9 @@ __global__ __launch_bounds__(kNmsThreads) void pp_nms_kernel(PPArgs p) {
     }
   }
   __syncthreads();
-  // exclusive scan of the class counts (ncls <= 1024), Hillis-Steele in soff
-  int v = tid < ncls ? scnt[tid] : 0;
-  soff[tid] = v;
-  __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {
-    const int add = tid >= d ? soff[tid - d] : 0;
-    __syncthreads();
-    soff[tid] += add;
-    __syncthreads();
-  }
-  soff[tid] -= v;  // inclusive -> exclusive
+  // exclusive scan of the class counts (ncls <= 1024)
+  const int v = tid < ncls ? scnt[tid] : 0;
+  soff[tid] = block_scan(v, wsum) - v;
   __syncthreads();
   // stable partition by class: one wave per class, ballots over the sorted order
   for (int c = wave; c < ncls; c += kNmsThreads / 64) {
@@ -316,27 +481,24 @@ __global__ __launch_bounds__(kNmsThreads) void pp_nms_kernel(PPArgs p) {
   const int q0 = tid * per, q1 = min(n, q0 + per);
   int mine = 0;
   for (int q = q0; q < q1; ++q) mine += (kbits[q >> 5] >> (q & 31)) & 1;
-  scnt[tid] = mine;
-  __syncthreads();
-  for (int d = 1; d < 1024; d <<= 1) {
-    const int add = tid >= d ? scnt[tid - d] : 0;
-    __syncthreads();
-    scnt[tid] += add;
-    __syncthreads();
+  const int upto = block_scan(mine, wsum);
+  if (tid == kNmsThreads - 1) {
+    const int first = atomicAdd(p.cursor, upto);
+    sn[2] = first;
+    cnt[0] = n;
+    cnt[1] = upto;
+    cnt[2] = 0;
+    cnt[3] = first;
   }
-  int k = scnt[tid] - mine;
+  __syncthreads();
+  int k = sn[2] + upto - mine;
   for (int q = q0; q < q1; ++q)
     if ((kbits[q >> 5] >> (q & 31)) & 1) {
       const int a = p.sorted_anchor[(size_t)b * nmax + q];
-      p.out_det[(size_t)b * nmax + k] = p.det[(size_t)b * A + a];
-      p.out_pos[(size_t)b * nmax + k] = q;
+      p.kept[k].det = p.det[(size_t)b * A + a];
+      p.kept[k].pos = q;
       ++k;
     }
-  if (tid == kNmsThreads - 1) {
-    cnt[0] = n;
-    cnt[1] = scnt[tid];
-    cnt[2] = 0;
-  }
 }
 
 }  // namespace
@@ -356,17 +518,30 @@ void launch_detect_tail(hipStream_t st, int dtype, const DetectTailArgs& t, floa
   }
   L.levels = t.levels;
   L.A = a;
-  const dim3 g((unsigned)((a + 255) / 256), (unsigned)n);
-  if (dtype == F16)
-    hipLaunchKernelGGL(detect_tail_kernel<true>, g, dim3(256), 0, st, L, out, t.nc, t.reg_max);
-  else if (dtype == F32)
-    hipLaunchKernelGGL(detect_tail_kernel<false>, g, dim3(256), 0, st, L, out, t.nc, t.reg_max);
-  else
-    fail(-2, "detect tail: f16 or f32 inputs");
+  if (dtype != F16 && dtype != F32) fail(-2, "detect tail: f16 or f32 inputs");
+  // The tile kernel reads dwords: f16 channels in pairs on 4-byte addresses,
+  // 64 anchors' dwords within its loads of 256 threads.
+  const int es = dtype == F16 ? 2 : 4, chans = 4 * t.reg_max + t.nc;
+  const size_t lds = ((size_t)kTailAnchors * (chans | 1) + 4 * kTailAnchors) * 4;
+  int tiles = 0;
+  bool tile = (chans * es) % 4 == 0 && chans * es / 4 * kTailAnchors <= tail_loads(dtype == F16) * 256;
+  for (int s = 0; s < t.levels; ++s) {
+    L.tile0[s] = tiles;
+    tiles += (t.h[s] * t.w[s] + kTailAnchors - 1) / kTailAnchors;
+    tile = tile && (t.pix[s] * es) % 4 == 0 && (uintptr_t)t.x[s] % 4 == 0;
+  }
+  if (tile) {
+    auto* k = dtype == F16 ? (t.reg_max == 16 ? detect_tail_tile_kernel<true, 16> : detect_tail_tile_kernel<true, 0>)
+                           : (t.reg_max == 16 ? detect_tail_tile_kernel<false, 16> : detect_tail_tile_kernel<false, 0>);
+    hipLaunchKernelGGL(k, dim3((unsigned)tiles, (unsigned)n), dim3(256), lds, st, L, out, t.nc, t.reg_max);
+  } else {
+    auto* k = dtype == F16 ? detect_tail_kernel<true> : detect_tail_kernel<false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)((a + 255) / 256), (unsigned)n), dim3(256), 0, st, L, out, t.nc, t.reg_max);
+  }
   DW_HIP(hipGetLastError());
 }
 
-size_t pp_nms_lds_bytes(int nmax) { return nms_lds_bytes(nmax); }
+size_t pp_nms_lds_bytes(int nmax) { return nms_lds_bytes(nmax) + kNmsThreads / 64 * sizeof(int); }
 
 void launch_yolo_postprocess(hipStream_t st, const PostprocessArgs& a) {
   PPArgs p{};
@@ -381,18 +556,15 @@ void launch_yolo_postprocess(hipStream_t st, const PostprocessArgs& a) {
   p.iou = a.iou;
   p.agnostic = a.agnostic;
   p.nmax = a.nmax;
-  int s = 1;
-  while (s < a.A) s <<= 1;
-  p.sort_n = s;
-  if ((size_t)s * 8 > (size_t)16 * a.nmax) fail(-2, "postprocess: too many anchors to sort");
+  if (a.A > 16384 || (size_t)16 * a.nmax < (size_t)16384 * 8) fail(-2, "postprocess: too many anchors to sort");
   if (a.nmax > kPPMaxCandidates) fail(-1, "postprocess: capacity");
   p.keys = a.keys;
   p.det = a.det;
   p.sorted_anchor = a.sorted_anchor;
   p.part_pos = a.part_pos;
-  p.out_det = a.out_det;
-  p.out_pos = a.out_pos;
+  p.kept = a.kept;
   p.counts = a.counts;
+  p.cursor = a.cursor;
   hipLaunchKernelGGL(pp_candidates_kernel, dim3((unsigned)((a.A + 255) / 256), (unsigned)a.n), dim3(256), 0, st,
                      p);
   DW_HIP(hipGetLastError());
