@@ -153,7 +153,7 @@ struct DirectArgs {
                            // round to f16 subnormals are checked in the kernel)
   int out_plain;           // 1: rint(x * out_rcp) == rint(x / out_scale) for every finite f16 x
   const float* wq;         // optional (f32 input, c_in % 16 == 0, c_out % 4 == 0): the weights as
-                           // [c_out / 4][kh * kw * c_in][4], for the tiled kernel
+                           // [c_out / 4][kh * kw * c_in][4], for the window kernel
   const float* wq16;       // optional (1x1, c_out % 16 == 0): the weights as [c_out / 16][c_in][16],
                            // for the 1x1 kernel's 16-channel groups
   int w_finite;            // 1: every weight is finite (the host that holds them checked), so an
@@ -290,6 +290,8 @@ void launch_direct_conv(hipStream_t st, const DirectArgs& a);
 // stride 2, pad 1, three dense f16 channels in, u8 out, finite weights;
 // DW_STEM_PAD=0 turns it off)
 bool stem_pad_ok(const DirectArgs& a);
+// true if a runs on the f32 window kernel once its weights are packed (wq)
+bool conv_window_f32_ok(const DirectArgs& a);
 bool conv1x1_u8_f16_supported(int cin, int cout);
 void launch_strided_copy(hipStream_t st, const StridedCopyArgs& a);
 void launch_broadcast_binary(hipStream_t st, const BinaryArgs& a);

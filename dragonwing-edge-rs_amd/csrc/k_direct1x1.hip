@@ -141,8 +141,8 @@ __global__ __launch_bounds__(64) void conv1x1_exact_kernel(const DirectArgs a) {
 }  // namespace
 
 bool launch_conv1x1_exact(hipStream_t st, const DirectArgs& a_in) {
-  if (a_in.kh != 1 || a_in.kw != 1 || a_in.pt != 0 || a_in.pl != 0) return false;
-  const int es = a_in.in_kind == 0 ? 4 : (a_in.in_kind == 1 ? 2 : 1);
+  if (a_in.in_kind == 0 || a_in.kh != 1 || a_in.kw != 1 || a_in.pt != 0 || a_in.pl != 0) return false;
+  const int es = a_in.in_kind == 1 ? 2 : 1;
   const int vn = 16 / es;
   if (a_in.cin % vn != 0 || (a_in.x_pix_stride * es) % 16 != 0 || (a_in.x_c_off * es) % 16 != 0 ||
       ((uintptr_t)a_in.x & 15) != 0)
@@ -195,7 +195,7 @@ bool launch_conv1x1_exact(hipStream_t st, const DirectArgs& a_in) {
     DW_HIP(hipGetLastError());                                                                      \
     return true;                                                                                    \
   }
-#define DW_K_ALL(CC, PP) DW_K(0, CC, PP, false) DW_K(1, CC, PP, false) DW_K(2, CC, PP, false) DW_K(2, CC, PP, true)
+#define DW_K_ALL(CC, PP) DW_K(1, CC, PP, false) DW_K(2, CC, PP, false) DW_K(2, CC, PP, true)
   DW_K_ALL(20, 4)
   DW_K_ALL(16, 4)
   DW_K_ALL(40, 2)
