@@ -31,7 +31,7 @@ def test_qconv_prep_bit_exact(backend, c_in, c_out, k):
     ys = float(0.02 * 4e-3 * 5000 * np.sqrt(c_in * k * k) / 40)
     bx, bw, bb = backend.from_numpy(x), backend.from_numpy(wt), backend.from_numpy(bias)
     by = backend.alloc(n * h * w * c_out)
-    for b, zp in ((bb, 131), (None, 3)):
+    for b, zp in ((bb, 131), (None, 3), (bb, 128), (None, 128)):
         ops.qlinearconv_u8s8(backend, bx, bw, b, by, n, h, w, c_in, c_out, k, k, 1, 1, p, p, 0.02, zp, ws, ys, 120)
         ref = oracle.qlinearconv_u8s8(x, wt, bias if b else None, (1, 1), (p, p), 0.02, zp, ws, ys, 120)
         np.testing.assert_array_equal(backend.to_numpy(by, np.uint8, (n, h, w, c_out)), ref)
