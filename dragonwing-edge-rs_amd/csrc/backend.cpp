@@ -465,11 +465,11 @@ static int dwconv_common(dw_hip_backend* be, int dtype, const dw_hip_buffer* inp
   std::lock_guard<std::mutex> lock(b->mu);
   const size_t es = dtype == DW_DTYPE_F16 ? 2 : 4;
   Geo g = geo(n, h_in, w_in, c, c, k_h, k_w, stride_h, stride_w, pad_h, pad_w);
-  // f16 3x3 with stride 1 or 2 runs on the sliding-window kernel (channel
+  // 3x3 with stride 1 or 2 runs on the row-marching kernel (in f16 with channel
   // groups of 4); every other shape on the generic one (groups of 8)
-  const bool sliding = dtype == DW_DTYPE_F16 && k_h == 3 && k_w == 3 && (stride_w == 1 || stride_w == 2);
-  if (c % (sliding ? 4 : 8) != 0)
-    dw::fail(DW_ERR_UNSUPPORTED, sliding ? "depthwise: c must be a multiple of 4" : "depthwise: c must be a multiple of 8");
+  const bool march = dtype == DW_DTYPE_F16 && k_h == 3 && k_w == 3 && (stride_w == 1 || stride_w == 2);
+  if (c % (march ? 4 : 8) != 0)
+    dw::fail(DW_ERR_UNSUPPORTED, march ? "depthwise: c must be a multiple of 4" : "depthwise: c must be a multiple of 8");
   need(input, n * h_in * w_in * c * es, "depthwise: input");
   need(kernel, k_h * k_w * c * es, "depthwise: kernel");
   need(output, n * g.ho * g.wo * c * es, "depthwise: output");

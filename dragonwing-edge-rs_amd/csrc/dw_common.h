@@ -238,7 +238,6 @@ struct DwArgs {
   int n, h, w, c, kh, kw, sh, sw, pt, pl, ho, wo;
   int act;
   int x_pix_stride, x_c_off, y_pix_stride, y_c_off;
-  int w_plain;  // 1: no f16 weight is subnormal (checked by whoever fills the struct)
 };
 
 // ---------------------------------------------------------------------------
@@ -301,6 +300,9 @@ void launch_conv1x1_u8_f16(hipStream_t st, const Conv1x1F16Args& a);
 // HWIO f32 weights [rows][cout] -> [cout / 4][rows][4] (DirectArgs::wq)
 void launch_repack_oc4(hipStream_t st, const float* w, float* wq, int rows, int cout);
 void launch_dwconv(hipStream_t st, const DwArgs& a, int dtype);
+// 3x3, stride 1 or 2 (k_dwconv3.hip); false, with nothing launched, if its
+// offsets or vector loads do not fit
+bool launch_dwconv3(hipStream_t st, const DwArgs& a, int dtype);
 // fp16 3x3 stride-1 depthwise on LDS row bands, packed f16 arithmetic (k_dwtile.hip)
 bool dwconv3_tile_ok(const DwArgs& a);
 bool dwconv3_tile_cfg_ok(const DwArgs& a, int units, int band_rows);

@@ -173,38 +173,7 @@ __device__ __forceinline__ uint2 conv1x1_f16_finish(f32x4 acc, const uint16_t* b
   return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
 }
 
-// acc + (f16 half SEL of x) * (f16 half SEL of w), fused, in f32: the f16
-// values widen exactly (subnormals at their IEEE value).  One v_fma_mix per
-// product; written out because the compiler otherwise widens reused
-// operands with separate conversions.
-template <int SEL>
-__device__ __forceinline__ float fma_mix_h(uint32_t x, uint32_t w, float acc) {
-  if constexpr (SEL == 0)
-    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[1,1,0]" : "+v"(acc) : "v"(x), "v"(w));
-  else
-    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "+v"(acc) : "v"(x), "v"(w));
-  return acc;
-}
-// (f16 half SEL of x) * (f16 half SEL of w) + 0: the first product of a
-// chain that starts at +0 (+0 + -0 is +0, as fma gives)
-template <int SEL>
-__device__ __forceinline__ float fma_mix_h0(uint32_t x, uint32_t w) {
-  float r;
-  if constexpr (SEL == 0)
-    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,1,0]" : "=v"(r) : "v"(x), "v"(w));
-  else
-    asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "=v"(r) : "v"(x), "v"(w));
-  return r;
-}
-// the same with an f32 weight
-template <int SEL>
-__device__ __forceinline__ float fma_mix_hf(uint32_t x, float w, float acc) {
-  if constexpr (SEL == 0)
-    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(x), "v"(w));
-  else
-    asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(x), "v"(w));
-  return acc;
-}
+// (f16 half SEL of x) * w + 0 in f32: the half widens in the instruction.
 template <int SEL>
 __device__ __forceinline__ float fma_mix_hf0(uint32_t x, float w) {
   float r;

@@ -12,7 +12,8 @@
 // 3-channel stem), and for the fp16 layers of the int8 graph that must match
 // the CPU bit for bit.
 //
-// dwconv: depthwise 3x3 (any k), channel multiplier 1.  One thread = one
+// dwconv: depthwise of any k and stride, channel multiplier 1 (3x3 at stride 1
+// or 2 is dwconv3_kernel's, k_dwconv3.hip).  One thread = one
 // pixel x 8 channels, so every load/store is a 16-byte (f16) or 32-byte
 // (f32) vector and consecutive threads walk consecutive channels (coalesced
 // NHWC).  No matrix cores: the op is HBM-bound.
@@ -517,204 +518,6 @@ __global__ __launch_bounds__(256) void stem_pad_u8_kernel(const DirectArgs a) {
   dx::store_outputs_t<2, 16, FE>(a, acc, oc0, (uint8_t*)a.y + yo, s_lut);
 }
 
-// Depthwise 3x3 over f16 NHWC.  A thread owns 4 channels of a block of
-// ROWS x SEG outputs; it loads the block's input window (NR rows of NC
-// columns, 8 bytes each) up front with buffer loads (a load outside the
-// tensor returns zeros; out-of-image rows and columns are sent out of range),
-// so every input is loaded (ROWS + 2) (SEG + 2) / (ROWS SEG) times at stride
-// 1 instead of 9.
-// Each output is the reference's sum: taps in (kh, kw) order, fmaf in f32.
-// The inputs enter the fma as f16 operands (v_fma_mix widens them exactly),
-// which is the reference's widening unless the value is an f16 subnormal
-// (the reference halves those): a wave in which any thread's window holds
-// one takes the decoding path for all its outputs.  WPLAIN: no weight is
-// subnormal (the planner checks), so the weights enter the fma as f16 too.
-// Out-of-image taps contribute an exact +0, which leaves the sum as the
-// reference's skip does (the running sum starts at +0 and so is never -0;
-// weights are finite).
-// Bias: the reference adds in f32 and rounds to f16; for f16 operands that
-// is the correctly rounded f16 sum (f32 holds 2 * 11 + 2 bits), so two
-// channels are added by one packed f16 add, unless the rounded sum or the
-// bias is an f16 subnormal (decoded at half value by the reference): then
-// the output takes the scalar decoding path.  SiLU: silu_f16_pk_lite (fp16
-// tolerance).  The buffer offsets are 32-bit: x spans at most 2^30 bytes,
-// so an offset plus BAD (2^30) is always past the buffer's x_bytes records.
-template <int SW, int SEG, int ROWS, bool WPLAIN, bool BIAS, int ACT>
-__global__ __launch_bounds__(256) void dwconv3_f16_kernel(const DwArgs a, int segs, int rblocks, int x_bytes) {
-  constexpr int CPT = 4;
-  constexpr int NC = SW * (SEG - 1) + 3;
-  constexpr int NR = SW * (ROWS - 1) + 3;
-  constexpr int BAD = 0x40000000;  // added to an offset below 2^30: out of range
-  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-  const int groups = a.c / CPT;
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= a.n * rblocks * segs * groups) return;
-  const int g = t % groups;
-  int rest = t / groups;
-  const int sg = rest % segs;
-  rest /= segs;
-  const int rb = rest % rblocks;
-  const int nn = rest / rblocks;
-  const int c0 = g * CPT;
-  const int ow0 = sg * SEG;
-  const int oh0 = rb * ROWS;
-
-  // weights and bias first: the first output needs them with its columns
-  uint2 wr[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) wr[k] = *reinterpret_cast<const uint2*>((const uint16_t*)a.wt + (size_t)k * a.c + c0);
-  uint2 br = make_uint2(0, 0);
-  if constexpr (BIAS) br = *reinterpret_cast<const uint2*>((const uint16_t*)a.bias + c0);
-
-  const __amdgpu_buffer_rsrc_t xrs =
-      __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, x_bytes, 0x00020000);
-  const int ps2 = a.x_pix_stride * 2;
-  int rowo[NR];
-#pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    const int ih = oh0 * a.sh - a.pt + r;
-    rowo[r] = (unsigned)ih < (unsigned)a.h ? ((nn * a.h + ih) * a.w) * ps2 + (a.x_c_off + c0) * 2 : BAD;
-  }
-  const int iw0 = ow0 * SW - a.pl;
-  int colo[NC];
-#pragma unroll
-  for (int q = 0; q < NC; ++q) colo[q] = (unsigned)(iw0 + q) < (unsigned)a.w ? (iw0 + q) * ps2 : BAD;
-  uint2 xc[NC][NR];
-#pragma unroll
-  for (int r = 0; r < NR; ++r)
-#pragma unroll
-    for (int q = 0; q < NC; ++q) {
-      const auto v = __builtin_amdgcn_raw_buffer_load_b64(xrs, rowo[r] + colo[q], 0, 0);
-      xc[q][r] = make_uint2(v[0], v[1]);
-    }
-
-  // any f16 subnormal in the window: (2|h| - 2) mod 2^16 < 0x7fe, both
-  // halves at once (one packed multiply-add, one packed min per register)
-  uint32_t mn = 0xffffffffu;
-  {
-    const uint32_t two = 0x00020002u, m2 = 0xfffefffeu;
-#pragma unroll
-    for (int r = 0; r < NR; ++r)
-#pragma unroll
-      for (int q = 0; q < NC; ++q) {
-        uint32_t t0, t1;
-        asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(t0) : "v"(xc[q][r].x), "v"(two), "s"(m2));
-        asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(t1) : "v"(xc[q][r].y), "v"(two), "s"(m2));
-        mn = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(us2, mn),
-                                                                    __builtin_bit_cast(us2, t0)));
-        mn = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(us2, mn),
-                                                                    __builtin_bit_cast(us2, t1)));
-      }
-  }
-  const bool sub_any = __any((mn & 0xffffu) < 0x7feu || (mn >> 16) < 0x7feu);
-
-  float wv[9][CPT];
-  if constexpr (!WPLAIN) {
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      wv[k][0] = h2f(wr[k].x & 0xffff);
-      wv[k][1] = h2f(wr[k].x >> 16);
-      wv[k][2] = h2f(wr[k].y & 0xffff);
-      wv[k][3] = h2f(wr[k].y >> 16);
-    }
-  }
-  const uint16_t bh[CPT] = {(uint16_t)(br.x & 0xffff), (uint16_t)(br.x >> 16), (uint16_t)(br.y & 0xffff),
-                            (uint16_t)(br.y >> 16)};
-  bool bias_sub = false;
-  if constexpr (BIAS) {
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) bias_sub |= (uint16_t)((bh[c] & 0x7fff) - 1) < 0x3ff;
-  }
-
-#define DW_HALVES(r_) {(uint16_t)((r_).x & 0xffff), (uint16_t)((r_).x >> 16), (uint16_t)((r_).y & 0xffff), (uint16_t)((r_).y >> 16)}
-#pragma unroll
-  for (int i = 0; i < ROWS; ++i) {
-    if (oh0 + i >= a.ho) break;
-    uint16_t* const yrow =
-        (uint16_t*)a.y + ((size_t)(nn * a.ho + oh0 + i) * a.wo) * a.y_pix_stride + a.y_c_off + c0;
-#pragma unroll
-    for (int j = 0; j < SEG; ++j) {
-      if (ow0 + j >= a.wo) break;
-      float acc[CPT] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (sub_any) {
-#pragma unroll
-        for (int kh = 0; kh < 3; ++kh)
-#pragma unroll
-          for (int kw = 0; kw < 3; ++kw) {
-            const uint16_t hv[CPT] = DW_HALVES(xc[SW * j + kw][SW * i + kh]);
-            const uint16_t hw[CPT] = DW_HALVES(wr[kh * 3 + kw]);
-#pragma unroll
-            for (int c = 0; c < CPT; ++c) {
-              const float wk = WPLAIN ? h2f_ieee(hw[c]) : wv[kh * 3 + kw][c];
-              acc[c] = fmaf(h2f(hv[c]), wk, acc[c]);
-            }
-          }
-      } else {
-#pragma unroll
-        for (int kh = 0; kh < 3; ++kh)
-#pragma unroll
-          for (int kw = 0; kw < 3; ++kw) {
-            const uint2 xv = xc[SW * j + kw][SW * i + kh];
-            const int k = kh * 3 + kw;
-            if constexpr (WPLAIN) {
-              if (k == 0) {
-                acc[0] = fma_mix_h0<0>(xv.x, wr[k].x);
-                acc[1] = fma_mix_h0<1>(xv.x, wr[k].x);
-                acc[2] = fma_mix_h0<0>(xv.y, wr[k].y);
-                acc[3] = fma_mix_h0<1>(xv.y, wr[k].y);
-              } else {
-                acc[0] = fma_mix_h<0>(xv.x, wr[k].x, acc[0]);
-                acc[1] = fma_mix_h<1>(xv.x, wr[k].x, acc[1]);
-                acc[2] = fma_mix_h<0>(xv.y, wr[k].y, acc[2]);
-                acc[3] = fma_mix_h<1>(xv.y, wr[k].y, acc[3]);
-              }
-            } else {
-              if (k == 0) {
-                acc[0] = fma_mix_hf0<0>(xv.x, wv[k][0]);
-                acc[1] = fma_mix_hf0<1>(xv.x, wv[k][1]);
-                acc[2] = fma_mix_hf0<0>(xv.y, wv[k][2]);
-                acc[3] = fma_mix_hf0<1>(xv.y, wv[k][3]);
-              } else {
-                acc[0] = fma_mix_hf<0>(xv.x, wv[k][0], acc[0]);
-                acc[1] = fma_mix_hf<1>(xv.x, wv[k][1], acc[1]);
-                acc[2] = fma_mix_hf<0>(xv.y, wv[k][2], acc[2]);
-                acc[3] = fma_mix_hf<1>(xv.y, wv[k][3], acc[3]);
-              }
-            }
-          }
-      }
-      // the conv result rounded to f16 (the reference's store)
-      h16x2 p01 = pk_f2h(acc[0], acc[1]), p23 = pk_f2h(acc[2], acc[3]);
-      if constexpr (BIAS) {
-        const float amin = fminf(fminf(fabsf(acc[0]), fabsf(acc[1])), fminf(fabsf(acc[2]), fabsf(acc[3])));
-        if (__any(bias_sub || amin < 6.103515625e-05f)) {
-          uint16_t hb[CPT] = {pk_lo(p01), pk_hi(p01), pk_lo(p23), pk_hi(p23)};
-#pragma unroll
-          for (int c = 0; c < CPT; ++c) hb[c] = f16_add_bits(hb[c], bh[c]);
-          p01 = pk_make(hb[0], hb[1]);
-          p23 = pk_make(hb[2], hb[3]);
-        } else {
-          p01 = p01 + __builtin_bit_cast(h16x2, br.x);
-          p23 = p23 + __builtin_bit_cast(h16x2, br.y);
-        }
-      }
-      if constexpr (ACT == ACT_SILU) {
-        p01 = silu_f16_pk_lite(p01);
-        p23 = silu_f16_pk_lite(p23);
-      } else if constexpr (ACT == ACT_RELU) {
-        uint16_t hb[CPT] = {pk_lo(p01), pk_hi(p01), pk_lo(p23), pk_hi(p23)};
-#pragma unroll
-        for (int c = 0; c < CPT; ++c) hb[c] = f16_act_bits(hb[c], ACT_RELU);
-        p01 = pk_make(hb[0], hb[1]);
-        p23 = pk_make(hb[2], hb[3]);
-      }
-      *reinterpret_cast<uint2*>(yrow + (size_t)(ow0 + j) * a.y_pix_stride) =
-          make_uint2(__builtin_bit_cast(uint32_t, p01), __builtin_bit_cast(uint32_t, p23));
-    }
-  }
-#undef DW_HALVES
-}
-
 template <int ESZ>
 __global__ __launch_bounds__(256) void dwconv_kernel(const DwArgs a) {
   constexpr int V = 8;
@@ -989,48 +792,9 @@ void launch_repack_oc4(hipStream_t st, const float* w, float* wq, int rows, int 
 }
 
 void launch_dwconv(hipStream_t st, const DwArgs& a, int dtype) {
-  // f16 3x3, stride 1 or 2: the sliding-window kernel (8-byte channel
-  // groups; the same sums, so the same results as the generic kernel)
-  const bool al8 = (uintptr_t)a.x % 8 == 0 && (uintptr_t)a.y % 8 == 0 && (uintptr_t)a.wt % 8 == 0 &&
-                   (uintptr_t)a.bias % 8 == 0 && (a.x_pix_stride * 2) % 8 == 0 && (a.x_c_off * 2) % 8 == 0 &&
-                   (a.y_pix_stride * 2) % 8 == 0 && (a.y_c_off * 2) % 8 == 0;
-  const long long x_bytes = ((long long)a.n * a.h * a.w - 1) * a.x_pix_stride * 2 + (a.x_c_off + a.c) * 2ll;
-  if (dtype == F16 && a.kh == 3 && a.kw == 3 && (a.sw == 1 || a.sw == 2) && a.sh == a.sw && a.c % 4 == 0 && al8 &&
-      x_bytes <= (1ll << 30)) {
-    // one row of 4 outputs per thread (3 x 6 input columns at stride 1, 3 x 9
-    // at stride 2): measured faster on 32 x 40 x 40 x 384 than 8 outputs, 2
-    // rows of 4 or 8, or an XCD-aware block order, whose larger windows
-    // cost occupancy and overlap between the loads and the arithmetic
-    constexpr int rows = 1;
-    const int seg = 4;
-    const int segs = (a.wo + seg - 1) / seg;
-    const int rblocks = (a.ho + rows - 1) / rows;
-    const long long threads = (long long)a.n * rblocks * segs * (a.c / 4);
-    if (threads < (1ll << 31)) {
-      const dim3 g((unsigned)((threads + 255) / 256));
-      const bool bias = a.bias != nullptr;
-#define DW_DW3(SW_, SEG_, WP_, B_, ACT_)                                                                    \
-  if (a.sw == SW_ && (a.w_plain != 0) == WP_ && bias == B_ && a.act == ACT_)                                 \
-    hipLaunchKernelGGL((dwconv3_f16_kernel<SW_, SEG_, rows, WP_, B_, ACT_>), g, dim3(256), 0, st, a, segs, \
-                       rblocks, (int)x_bytes);                                                             \
-  else
-#define DW_DW3_ACTS(SW_, SEG_, WP_, B_) \
-  DW_DW3(SW_, SEG_, WP_, B_, ACT_NONE) DW_DW3(SW_, SEG_, WP_, B_, ACT_RELU) DW_DW3(SW_, SEG_, WP_, B_, ACT_SILU)
-      DW_DW3_ACTS(1, 4, true, true)
-      DW_DW3_ACTS(1, 4, true, false)
-      DW_DW3_ACTS(1, 4, false, true)
-      DW_DW3_ACTS(1, 4, false, false)
-      DW_DW3_ACTS(2, 4, true, true)
-      DW_DW3_ACTS(2, 4, true, false)
-      DW_DW3_ACTS(2, 4, false, true)
-      DW_DW3_ACTS(2, 4, false, false)
-      fail(-2, "depthwise: no kernel for this activation");
-#undef DW_DW3_ACTS
-#undef DW_DW3
-      DW_HIP(hipGetLastError());
-      return;
-    }
-  }
+  // 3x3 at stride 1 or 2 (the same sums, so the same results as the generic
+  // kernel)
+  if (launch_dwconv3(st, a, dtype)) return;
   if (a.c % 8 != 0) fail(-2, "depthwise: c must be a multiple of 8 for this shape");
   const size_t total = (size_t)a.n * a.ho * a.wo * (a.c / 8);
   size_t blocks = (total + 255) / 256;

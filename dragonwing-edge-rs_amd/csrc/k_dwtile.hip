@@ -1,6 +1,6 @@
 // Depthwise 3x3 convolution, stride 1, padding 1, fp16 NHWC, with bias and
 // activation, held to the fp16 tolerance: the bandwidth-bound path of the
-// fp16 graphs.  (dwconv3_f16_kernel in k_direct.hip is the reference-order
+// fp16 graphs.  (dwconv3_kernel in k_dwconv3.hip is the reference-order
 // alternative, bit-exact before the activation.)
 //
 // A workgroup owns one image, a band of RB output rows, every column and a
