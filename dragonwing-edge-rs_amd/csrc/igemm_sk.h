@@ -260,16 +260,7 @@ __global__ __launch_bounds__(256) void igemm_sk_kernel(const IgemmArgs a) {
         }
       }
     } else {
-#pragma unroll
-      for (int cb = 0; cb < CB; ++cb) {
-        const int ch = c0 + cb * 16 + cq;
-        if (ch >= a.cout) continue;
-#pragma unroll
-        for (int pb = 0; pb < PB; ++pb) {
-          const int p = pc + pb * 16 + (lane & 15);
-          if (p < a.m) epilogue4<ESZ>(a, ep, acc[cb][pb], ch, ch - c0, p);
-        }
-      }
+      igemm_store<ESZ, BC, PB, EPV>(a, ep, acc, c0, pc, lane, s_ms, s_lut);
     }
     if (!more) break;
   }
