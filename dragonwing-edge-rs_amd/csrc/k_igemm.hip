@@ -5,6 +5,7 @@
 // igemm_wide.h); their instantiations live in the k_igemm_*.hip files so
 // that they compile in parallel.
 #include "igemm_band.h"
+#include "igemm_fp.h"
 #include "igemm_ks.h"
 #include "igemm_rows.h"
 #include "igemm_sk.h"
@@ -326,6 +327,22 @@ TileCfg make_ks_tile(const IgemmArgs& a, int bc, int waves) {
   return t;
 }
 
+// The in-order fp16 kernel (tpw = -7): 16, 32 or 64 channels of 16 pixels, taps
+// of whole k-steps.
+bool fp_ok(const IgemmArgs& a, int bc) {
+  return a.epi == EPI_F16 && !a.h_wfrag && (bc == 16 || bc == 32 || bc == 64) && a.cout_pad % bc == 0 &&
+         a.cin % 32 == 0;
+}
+
+// Its tiles that are few: at most a wave a SIMD.
+bool fp_few(const IgemmArgs& a, int bc) { return (long)((a.m + 15) / 16) * (a.cout_pad / bc) <= 1024; }
+
+TileCfg make_fp_tile(const IgemmArgs& a, int bc) {
+  TileCfg t = make_tile(a, bc, 1);
+  t.tpw = -7;
+  return t;
+}
+
 // A detect head's 1x1 fused into the epilogue (a.h_wfrag): one tile holds
 // every channel (64 or 80) on the staged kernel (with room for the regroup
 // rows in its weight chunk), the row-tile or the band-tile kernel.
@@ -382,6 +399,15 @@ float ks_cost(const IgemmArgs& a, int bc, int waves) {
          full * (0.05115f * batches + 0.0971f * nw);
 }
 
+// The same for the in-order fp16 kernel (fit to 63 timings, 10%): its chain of
+// k-steps, shorter where up to four share their addresses, and the CUs' loads.
+float fp_cost(const IgemmArgs& a, int bc) {
+  const long waves = (long)((a.m + 15) / 16) * (a.cout_pad / bc);
+  const float mean = (float)waves / 256.0f, full = (float)((waves + 255) / 256);
+  const float ks = (float)a.ksteps, cb = (float)bc / 16.0f, shared = a.cin % 128 == 0 ? 4.0f : a.cin % 64 == 0 ? 2.0f : 1.0f;
+  return 3.367f + 0.0554f * ks / shared + mean * (0.4539f + 0.0518f * cb + 0.01781f * ks) + 0.01207f * full * ks * cb;
+}
+
 // Tile shape for a problem: an override from DW_IGEMM_TILE (tests and
 // tuning runs), an explicit choice (a.tile_bc / a.tile_pb, set by the graph
 // runtime's tuner), else the tile that tile_cost expects to be fastest.  The
@@ -431,6 +457,7 @@ TileCfg pick_any(const IgemmArgs& a) {
     if (nv == 3 && v2 == -3 && wide_ok(a, v0)) return make_wide_tile(a, v0);
     if (nv == 3 && (v2 == -4 || v2 == -5) && band_ok(a, v0, v1, v2)) return make_band_tile(a, v0, v1, v2);
     if (nv == 3 && v2 == -6 && ks_ok(a, v0, v1)) return make_ks_tile(a, v0, v1);
+    if (nv == 3 && v2 == -7 && fp_ok(a, v0)) return make_fp_tile(a, v0);
     if (nv >= 2 && tile_ok(a, v0, v1)) return make_tile(a, v0, v1);
     if (nv == 1 && tile_ok(a, channel_tile(a.cout), v0)) return make_tile(a, channel_tile(a.cout), v0);
   }
@@ -441,6 +468,7 @@ TileCfg pick_any(const IgemmArgs& a) {
   if (a.tile_bc && (a.tile_tpw == -4 || a.tile_tpw == -5) && band_ok(a, a.tile_bc, a.tile_pb, a.tile_tpw))
     return make_band_tile(a, a.tile_bc, a.tile_pb, a.tile_tpw);
   if (a.tile_bc && a.tile_tpw == -6 && ks_ok(a, a.tile_bc, a.tile_pb)) return make_ks_tile(a, a.tile_bc, a.tile_pb);
+  if (a.tile_bc && a.tile_tpw == -7 && fp_ok(a, a.tile_bc)) return make_fp_tile(a, a.tile_bc);
   if (a.tile_bc && tile_ok(a, a.tile_bc, a.tile_pb)) return make_tile(a, a.tile_bc, a.tile_pb);
   // The widest channel tile and the widest pixel tile (16 * pb pixels per
   // wave) that still gives about two workgroups per CU reads the input least
@@ -491,6 +519,17 @@ TileCfg pick_any(const IgemmArgs& a) {
           best = make_ks_tile(a, b, nw);
         }
       }
+  // fp16 on few pixels: half of the 29 layers of up to 1024 such waves, those
+  // 1.37x faster; below four k-steps there is no chain to shorten (7 x 21 96
+  // -> 92 1x1 of 5 images: 4.8 against 3.9 us)
+  for (int b : {16, 32, 64})
+    if (a.ksteps >= 4 && fp_ok(a, b) && fp_few(a, b)) {
+      const float c = fp_cost(a, b);
+      if (c < least) {
+        least = c;
+        best = make_fp_tile(a, b);
+      }
+    }
   return best;
 }
 
@@ -512,8 +551,8 @@ bool igemm_sibling_tile_ok(const IgemmArgs& a, int bc, int tpw, int esize) {
   if (esize == 1)  // the u8 table epilogue (its table staged per channel tile)
     return common && a.epi == EPI_QU8 && a.lut && a.lut2 &&
            (tpw == 0 || tpw == -1 || tpw == -4 || tpw == -5 || tpw == -6);
-  // fp16: the generic epilogue chooses the view per four channels; every
-  // kernel storing through igemm_store (not the persistent small-K kernel)
+  // fp16: the store chooses the view per channel tile; every kernel but the
+  // persistent small-K one
   return common && esize == 2 && a.epi == EPI_F16 && tpw <= 0;
 }
 
@@ -552,6 +591,13 @@ int igemm_candidates(const IgemmArgs& a, int* bc, int* pb, int* tpw, int max) {
         tpw[n] = -6;
         ++n;
       }
+  for (int b : {16, 32, 64})
+    if (n < max && fp_ok(a, b) && fp_few(a, b)) {
+      bc[n] = b;
+      pb[n] = 1;
+      tpw[n] = -7;
+      ++n;
+    }
   // band tiles (8 and 16 waves): the widest channel tile, and 64 or 80
   // channels when that splits a wider layer in two or more (80: a sibling
   // GEMM whose first conv has 80 channels)
@@ -628,6 +674,8 @@ const char* igemm_tile_name(const IgemmArgs& a, int esize) {
     snprintf(buf, sizeof buf, "igemm_%s_c%d_band%dw16", esize == 1 ? "i8" : "f16", t.bc, t.pb);
   else if (t.tpw == -6)
     snprintf(buf, sizeof buf, "igemm_%s_c%d_ks%d", esize == 1 ? "i8" : "f16", t.bc, t.pb);
+  else if (t.tpw == -7)
+    snprintf(buf, sizeof buf, "igemm_%s_c%d_fp", esize == 1 ? "i8" : "f16", t.bc);
   else
     snprintf(buf, sizeof buf, "igemm_%s_c%d_p%d", esize == 1 ? "i8" : "f16", t.bc, 64 * t.pb);
   if (a.h_wfrag) strncat(buf, "_head", sizeof buf - strlen(buf) - 1);
@@ -652,7 +700,7 @@ void launch_igemm(hipStream_t st, const IgemmArgs& a_in, int esize) {
                      : t.tpw == -3 ? ig::wide_lds_bytes(t.bc, a.ksteps)
                      : t.tpw == -4 || t.tpw == -5
                          ? ig::band_lds_bytes(t.bc, a.ksteps, t.pb, a.wo, a.cin * esize / 16, band_waves(t.tpw), a.sh)
-                     : t.tpw == -6 ? 0
+                     : t.tpw <= -6 ? 0
                                    : ig::lds_bytes(t, a.ksteps);
   if (lds > 160 * 1024) fail(-2, "igemm: k-slice table does not fit LDS");
   if ((long long)a.ho * a.wo >= (1ll << 23)) fail(-2, "igemm: more than 2^23 output pixels per image");
@@ -706,6 +754,7 @@ void launch_igemm(hipStream_t st, const IgemmArgs& a_in, int esize) {
          : t.tpw == -1 ? igemm_launch_st_f16(st, a, t)
          : t.tpw == -2 ? igemm_launch_rows_f16(st, a, t)
          : t.tpw == -3 ? igemm_launch_wide_f16(st, a, t)
+         : t.tpw == -7 ? igemm_launch_fp_f16(st, a, t)
          : t.tpw == -4 || t.tpw == -5 ? igemm_launch_band_f16(st, a, t)
                        : igemm_launch_f16(st, a, t);
   }
