@@ -360,38 +360,35 @@ bool head_tile_ok(const IgemmArgs& a, const TileCfg& t) {
 // the workgroups costs in matrix instructions, im2col loads, weight reads and
 // epilogues per k-step, with the share both as the mean (tiles / 256) and as
 // the busiest CU's whole tiles.  The coefficients are a non-negative least
-// squares fit (relative error 8-12%) to 10,600 timings of 810 convolutions
-// with 1-32 images of 7-160 rows and columns, 16-512 input and 16-1000
-// output channels, 1x1 and 3x3, strides 1 and 2.
-float tile_cost(const IgemmArgs& a, const TileCfg& t, int esize) {
+// squares fit (relative error 8-12%) to the timings of 475 int8 and 337 fp16
+// convolutions with 1-32 images of 7-160 rows and columns, 16-512 input and
+// 16-1000 output channels, 1x1 and 3x3, strides 1 and 2.  Choosing among up to
+// 50 tiles is host time of every untimed launch, so the arguments are what
+// the candidates share: 0.3 us (0.9-2.2 us with each tile laid out first).
+float tile_cost(int esize, int fam, int ksteps, int bc, int pb, int wgs) {
   static const float kFit[2][3][15] = {
       {{3.254f, 0.1118f, 0.003944f, 0.01639f, 0.002887f, 0.04835f, 0.08821f, 0.002636f, 0.0154f, 0, 0.01487f,
         0.002478f, 0.01127f, 0.01528f, 0.08366f},
        {3.93f, 0.08103f, 0, 0.01531f, 0, 0.06327f, 0.5737f, 0.002326f, 0, 0, 0, 0.0008586f, 0.04129f, 0.01257f,
         0.1047f},
        {3.394f, 0, 0, 0, 0, 0, 1.221f, 0.00399f, 0, 0, 0, 0.006569f, 0.05407f, 0, 0.08989f}},
-      {{3.111f, 0.1012f, 0.003483f, 0, 0, 0.1107f, 0.01602f, 0.003486f, 0.01775f, 0, 0.04173f, 0.008584f, 0.01336f,
-        0.01142f, 0.05833f},
-       {3.456f, 0.09272f, 0, 0, 0, 0.06695f, 0.6392f, 0.002246f, 0.00824f, 0, 0, 0.003731f, 0.03211f, 0.007329f,
-        0.1647f},
-       {2.013f, 0, 0, 0, 0, 0, 1.174f, 0.003609f, 0, 0, 0.008598f, 0.005149f, 0.04719f, 0, 0.1771f}}};
-  const int fam = t.tpw == -3 ? 2 : t.tpw == -1 ? 1 : 0;
-  const long wgs = (long)((a.m + 64 * t.pb - 1) / (64 * t.pb)) * (a.cout_pad / t.bc);
-  const float ks = (float)a.ksteps, b = (float)t.bc / 16.0f, p = (float)t.pb;
-  const float mean = (float)wgs / 256.0f, full = (float)((wgs + 255) / 256);
-  const float f[15] = {1,           ks,          ks * b,         ks * p,        ks * b * p,
-                       b * p,       mean,        mean * ks * b * p, mean * ks * p, mean * ks * b,
-                       mean * b * p, full * ks * b * p, full * ks * p, full * ks * b, full * b * p};
+      {{3.626f, 0.07469f, 0.005534f, 0, 0.003169f, 0.01053f, 0.0151f, 0.001067f, 0.01693f, 0, 0.06502f,
+        0.004994f, 0.02329f, 0.01432f, 0.03708f},
+       {3.885f, 0.0769f, 0, 0, 0, 0, 0.5448f, 0.002746f, 0.009312f, 0, 0, 0.003492f, 0.03948f, 0.01009f, 0.1019f},
+       {3.033f, 0, 0, 0, 0, 0, 1.406f, 0.002105f, 0, 0, 0.04805f, 0.008186f, 0.03759f, 0, 0.05602f}}};
+  const float ks = (float)ksteps, b = (float)bc / 16.0f, p = (float)pb;
+  const float kb = ks * b, kp = ks * p, bp = b * p, kbp = kb * p;
+  const float mean = (float)wgs * (1.0f / 256.0f), full = (float)((wgs + 255) >> 8);
   const float* c = kFit[esize == 1 ? 0 : 1][fam];
-  float cost = 0;
-  for (int i = 0; i < 15; ++i) cost += c[i] * f[i];
-  return cost;
+  const float one = (c[0] + c[1] * ks) + (c[2] * kb + c[3] * kp) + (c[4] * kbp + c[5] * bp);
+  const float share = c[6] + (c[7] * kbp + c[8] * kp) + (c[9] * kb + c[10] * bp);
+  const float busiest = (c[11] * kbp + c[12] * kp) + (c[13] * kb + c[14] * bp);
+  return one + mean * share + full * busiest;
 }
 
 // The same for the split-K kernel of `waves` waves (fit to 493 timings, 6%):
 // its batches of loads, and the busiest CU's waves and batches.
-float ks_cost(const IgemmArgs& a, int bc, int waves) {
-  const long wgs = (long)((a.m + 15) / 16) * (a.cout_pad / bc);
+float ks_cost(const IgemmArgs& a, int bc, int waves, int wgs) {
   const float mean = (float)wgs / 256.0f, full = (float)((wgs + 255) / 256), nw = (float)waves;
   const int per = (a.ksteps + waves - 1) / waves;
   const float batches = (float)((per + ig::kKsAhead - 1) / ig::kKsAhead);
@@ -401,8 +398,7 @@ float ks_cost(const IgemmArgs& a, int bc, int waves) {
 
 // The same for the in-order fp16 kernel (fit to 63 timings, 10%): its chain of
 // k-steps, shorter where up to four share their addresses, and the CUs' loads.
-float fp_cost(const IgemmArgs& a, int bc) {
-  const long waves = (long)((a.m + 15) / 16) * (a.cout_pad / bc);
+float fp_cost(const IgemmArgs& a, int bc, int waves) {
   const float mean = (float)waves / 256.0f, full = (float)((waves + 255) / 256);
   const float ks = (float)a.ksteps, cb = (float)bc / 16.0f, shared = a.cin % 128 == 0 ? 4.0f : a.cin % 64 == 0 ? 2.0f : 1.0f;
   return 3.367f + 0.0554f * ks / shared + mean * (0.4539f + 0.0518f * cb + 0.01781f * ks) + 0.01207f * full * ks * cb;
@@ -474,9 +470,9 @@ TileCfg pick_any(const IgemmArgs& a) {
   // wave) that still gives about two workgroups per CU reads the input least
   // often, but leaves CUs idle on small maps and makes long workgroups of
   // deep layers; it stays unless another tile is expected to take under 95%
-  // of its time.  On 270 convolutions kept out of the fit the choice is 1.17x
-  // faster (geometric mean) and 4.5% off the best tile; 1% of them are more
-  // than 3% slower, the worst 7%.  20 x 20, 256 -> 256 3x3, one image: 15.8
+  // of its time.  On 250 convolutions kept out of the fits the choice is 1.16x
+  // faster (geometric mean) and 4.3% off the best tile; 1-2% of them are more
+  // than 3% slower, the worst 9%.  20 x 20, 256 -> 256 3x3, one image: 15.8
   // -> 9.2 us.
   const int bc = channel_tile(a.cout);
   const int ctiles = a.cout_pad / bc;
@@ -490,47 +486,58 @@ TileCfg pick_any(const IgemmArgs& a) {
   }
   if (a.y2 || a.y_up) return best;  // the graph runtime's fused launches
   const int esize = a.epi == EPI_F16 ? 2 : 1;
-  float least = 0.95f * tile_cost(a, best, esize);
-  auto consider = [&](const TileCfg& t) {
-    const float c = tile_cost(a, t, esize);
+  // 64 PB-pixel tiles: (m + 64 PB - 1) / (64 PB) for PB = 1, 2, 4
+  auto pixel_tiles = [&](int pb) { return (a.m + 64 * pb - 1) >> (pb == 4 ? 8 : pb == 2 ? 7 : 6); };
+  float least = 0.95f * tile_cost(esize, 0, a.ksteps, best.bc, best.pb, pixel_tiles(best.pb) * ctiles);
+  int b_bc = 0, b_pb = 0, b_tpw = 0;  // the best so far, if not `best`
+  auto consider = [&](float c, int b, int p, int tpw) {
     if (c < least) {
       least = c;
-      best = t;
+      b_bc = b;
+      b_pb = p;
+      b_tpw = tpw;
     }
   };
-  for (int b : {128, 96, 80, 64, 48, 32, 16})
+  for (int b : {128, 96, 80, 64, 48, 32, 16}) {
+    if (b > bc || a.cout_pad % b != 0) continue;  // tile_ok, for each pixel tile
+    const int ct = a.cout_pad / b;
     for (int p : {4, 2, 1}) {
-      if (tile_ok(a, b, p)) consider(make_tile(a, b, p));
-      if (st_ok(a, b, p)) consider(make_st_tile(a, b, p));
+      const int wgs = pixel_tiles(p) * ct;
+      consider(tile_cost(esize, 0, a.ksteps, b, p, wgs), b, p, 0);
+      if (a.ksteps >= 2 && ig::st_lds_bytes(b, a.ksteps, ring_depth(p)) <= 160 * 1024)  // st_ok
+        consider(tile_cost(esize, 1, a.ksteps, b, p, wgs), b, p, -1);
     }
+  }
   for (int b : {256, 128, 64})
-    if (wide_ok(a, b)) consider(make_wide_tile(a, b));
-  // Split K on few pixels (int8: a sum of integers is the same in any order;
-  // fp16 layers keep one order for every plan): a fifth of the int8 layers
-  // above, those 1.30x faster, and the best tile 4.6% away instead of 11%.
-  // 20 x 20, 256 -> 256 3x3, one image: 9.2 -> 5.5 us.
-  least = std::min(least, 0.95f * tile_cost(a, best, esize));
-  for (int b : {16, 32})
-    for (int nw : {4, 8, 16})
-      if (ks_ok(a, b, nw) && ks_few(a, b)) {
-        const float c = ks_cost(a, b, nw);
-        if (c < least) {
-          least = c;
-          best = make_ks_tile(a, b, nw);
-        }
-      }
-  // fp16 on few pixels: half of the 29 layers of up to 1024 such waves, those
-  // 1.37x faster; below four k-steps there is no chain to shorten (7 x 21 96
-  // -> 92 1x1 of 5 images: 4.8 against 3.9 us)
-  for (int b : {16, 32, 64})
-    if (a.ksteps >= 4 && fp_ok(a, b) && fp_few(a, b)) {
-      const float c = fp_cost(a, b);
-      if (c < least) {
-        least = c;
-        best = make_fp_tile(a, b);
-      }
+    if (wide_ok(a, b)) consider(tile_cost(esize, 2, a.ksteps, b, 4, pixel_tiles(4) * (a.cout_pad / b)), b, 4, -3);
+  // Tiles of 16 pixels where they are few, against 95% of the best above
+  // (least when nothing above was chosen is that already).
+  // Split K (int8: a sum of integers is the same in any order; fp16 layers
+  // keep one order for every plan): a fifth of the int8 layers above, those
+  // 1.30x faster, and the best tile 4.6% away instead of 11%.  20 x 20, 256 ->
+  // 256 3x3, one image: 9.2 -> 5.5 us.
+  // In order (fp16): half of 29 layers of up to 1024 such waves, those 1.37x
+  // faster; below four k-steps there is no chain to shorten (7 x 21 96 -> 92
+  // 1x1 of 5 images: 4.8 against 3.9 us).
+  if (b_bc) least *= 0.95f;
+  const int p16 = (a.m + 15) >> 4;
+  for (int b : {16, 32, 64}) {
+    if (a.cout_pad % b != 0) continue;
+    const long tiles = (long)p16 * (a.cout_pad / b);
+    if (tiles > 1024) continue;  // ks_few, fp_few
+    if (esize == 2) {
+      if (a.ksteps >= 4 && fp_ok(a, b)) consider(fp_cost(a, b, (int)tiles), b, 1, -7);
+    } else {
+      for (int nw : {4, 8, 16})
+        if (ks_ok(a, b, nw)) consider(ks_cost(a, b, nw, (int)tiles), b, nw, -6);
     }
-  return best;
+  }
+  if (!b_bc) return best;
+  return b_tpw == 0    ? make_tile(a, b_bc, b_pb)
+         : b_tpw == -1 ? make_st_tile(a, b_bc, b_pb)
+         : b_tpw == -3 ? make_wide_tile(a, b_bc)
+         : b_tpw == -6 ? make_ks_tile(a, b_bc, b_pb)
+                       : make_fp_tile(a, b_bc);
 }
 
 // Epilogue specialisation for the arguments.
