@@ -331,7 +331,7 @@ TileCfg make_ks_tile(const IgemmArgs& a, int bc, int waves) {
 // of whole k-steps.
 bool fp_ok(const IgemmArgs& a, int bc) {
   return a.epi == EPI_F16 && !a.h_wfrag && (bc == 16 || bc == 32 || bc == 64) && a.cout_pad % bc == 0 &&
-         a.cin % 32 == 0;
+         a.cin % 32 == 0 && a.ksteps == a.kh * a.kw * (a.cin / 32);
 }
 
 // Its tiles that are few: at most a wave a SIMD.
