@@ -85,7 +85,7 @@ hipError_t Backend::copy_chunks(uint8_t* dst, const uint8_t* src, size_t bytes, 
   return err;
 }
 
-// Through the page-locked slots: the driver's own copy to ordinary memory
+// Through the page-locked slots: HIP's own copy to ordinary memory
 // runs at 18 GB/s, and one to page-locked memory at 56 GB/s of which a thread
 // moves 31 GB/s on (less into pages touched for the first time), so from 4 MiB
 // on four threads copy.  Measured into warm memory: 0.46 MB 37 us, 1.8 MB 90
