@@ -6,10 +6,14 @@
 #include "dw_common.h"
 #include "dw_device.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace dw {
 namespace {
+
+// Workgroups of up to 256 threads in x: HIP refuses 2^32 threads or more there.
+constexpr long long kMaxGridX = 1 << 23;
 
 // C[i][j] = sum over p of A[i][p] * B[p][j].  f32: fma chain from +0 in p
 // order (gemm_f32_naive, ops.rs:273-290).  F16: operands widened with the
@@ -41,8 +45,9 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_exact_kernel(const void* A,
   using E = std::conditional_t<F16, uint16_t, float>;
   const E* a = (const E*)A;
   const E* b = (const E*)B;
-  const unsigned t = threadIdx.x, i0 = blockIdx.y * kGemmR, j0 = blockIdx.x * kGemmC;
+  const unsigned t = threadIdx.x, i0 = blockIdx.y * kGemmR, j0 = (blockIdx.z * gridDim.x + blockIdx.x) * kGemmC;
   const unsigned um = m, un = n, uk = k;
+  if (j0 >= un) return;  // the last grid z's workgroups past the columns
   const unsigned lr = t / kGemmC, lc = t % kGemmC;  // the thread's output; (k quad, column) when it loads B
   auto widen = [](E v) -> float {
     if constexpr (F16) return h2f(v);
@@ -211,9 +216,11 @@ __device__ __forceinline__ float group_reduce(float v, Op op) {
 constexpr int kSoftmaxRegs = 8;
 template <bool H, int G>
 __global__ __launch_bounds__(256) void softmax_rows_kernel(const void* X, void* Y, int rows, int n) {
-  const int r = (int)blockIdx.x * (256 / G) + (int)threadIdx.x / G, l = threadIdx.x % G;
-  const bool live = r < rows;  // a dead group runs along (its lanes' wave reduces together)
-  const size_t base = (size_t)(live ? r : 0) * n;
+  // (grid y: a launch's threads in x stay below 2^32)
+  const size_t r = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * (256 / G) + threadIdx.x / G;
+  const int l = threadIdx.x % G;
+  const bool live = r < (size_t)rows;  // a dead group runs along (its lanes' wave reduces together)
+  const size_t base = (live ? r : 0) * n;
   auto ld = [&](int i) -> float {
     if constexpr (H) return h2f(((const uint16_t*)X)[base + i]);
     return ((const float*)X)[base + i];
@@ -337,7 +344,8 @@ __global__ __launch_bounds__(256) void transpose_u8_kernel(const uint8_t* src, u
 void launch_gemm_ex(hipStream_t st, int dtype, const void* a, const void* b, void* c, int m, int n, int k,
                     bool trans_b, const void* bias, int blen) {
   if (m > 65535) fail(-2, "gemm: more than 65535 rows");
-  const dim3 g((unsigned)(((long long)n + kGemmC - 1) / kGemmC), (unsigned)((m + kGemmR - 1) / kGemmR));
+  const long long cols = ((long long)n + kGemmC - 1) / kGemmC, gx = std::min(cols, kMaxGridX);
+  const dim3 g((unsigned)gx, (unsigned)((m + kGemmR - 1) / kGemmR), (unsigned)((cols + gx - 1) / gx));
   if (dtype == F32 && !trans_b)
     hipLaunchKernelGGL((gemm_exact_kernel<false, false>), g, dim3(kGemmThreads), 0, st, a, b, c, m, n, k, bias, blen);
   else if (dtype == F32)
@@ -378,20 +386,29 @@ void launch_softmax_rows(hipStream_t st, const float* x, float* y, int rows, int
   launch_softmax_rows_t(st, F32, x, y, rows, n);
 }
 
+namespace {
 // The smallest group that keeps a row in registers: a DFL's 16 bins take 16
 // threads (four rows a wave), a classifier's 1000 classes a workgroup.
-void launch_softmax_rows_t(hipStream_t st, int dtype, const void* x, void* y, int rows, int n) {
-  if (dtype != F32 && dtype != F16) fail(-2, "softmax: dtype");
+template <bool H>
+void launch_softmax(hipStream_t st, const void* x, void* y, int rows, int n) {
   const int g = n <= kSoftmaxRegs * 16 ? 16 : n <= kSoftmaxRegs * 64 ? 64 : 256;
-  const dim3 grid((unsigned)(((long long)rows * g + 255) / 256));
-  auto* k = dtype == F16 ? (g == 16   ? softmax_rows_kernel<true, 16>
-                            : g == 64 ? softmax_rows_kernel<true, 64>
-                                      : softmax_rows_kernel<true, 256>)
-                         : (g == 16   ? softmax_rows_kernel<false, 16>
-                            : g == 64 ? softmax_rows_kernel<false, 64>
-                                      : softmax_rows_kernel<false, 256>);
-  hipLaunchKernelGGL(k, grid, dim3(256), 0, st, x, y, rows, n);
+  auto* k = g == 16   ? softmax_rows_kernel<H, 16>
+            : g == 64 ? softmax_rows_kernel<H, 64>
+                      : softmax_rows_kernel<H, 256>;
+  const long long blocks = ((long long)rows * g + 255) / 256;
+  const long long gx = std::min(blocks, kMaxGridX);
+  hipLaunchKernelGGL(k, dim3((unsigned)gx, (unsigned)((blocks + gx - 1) / gx)), dim3(256), 0, st, x, y, rows, n);
   DW_HIP(hipGetLastError());
+}
+}  // namespace
+
+void launch_softmax_rows_t(hipStream_t st, int dtype, const void* x, void* y, int rows, int n) {
+  if (dtype == F32)
+    launch_softmax<false>(st, x, y, rows, n);
+  else if (dtype == F16)
+    launch_softmax<true>(st, x, y, rows, n);
+  else
+    fail(-2, "softmax: dtype");
 }
 
 }  // namespace dw
