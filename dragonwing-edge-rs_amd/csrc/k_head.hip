@@ -185,7 +185,7 @@ __global__ __launch_bounds__(64) void global_avg_pool_kernel(const void* X, void
     ((float*)Y)[(size_t)b * c + ch] = mean;
 }
 
-// Reductions over a group of G consecutive threads (G = 16, 64: lanes of a
+// Reductions over a group of G consecutive threads (G up to 64: lanes of a
 // wave; 256: the workgroup, through LDS).
 template <int G, typename Op>
 __device__ __forceinline__ float group_reduce(float v, Op op) {
@@ -387,12 +387,18 @@ void launch_softmax_rows(hipStream_t st, const float* x, float* y, int rows, int
 }
 
 namespace {
-// The smallest group that keeps a row in registers: a DFL's 16 bins take 16
-// threads (four rows a wave), a classifier's 1000 classes a workgroup.
+// Four values a thread up to a row of 16, which many short rows ask for (the
+// kernel's time is its slots then: 262144 rows of 1 value 3.7 us with a
+// thread a row, 19.6 us with 16; of 8, 6.6 us with 2, 20.5 us with 16; of 16,
+// 8.5 us with 4, 20.6 us with 16); beyond, the smallest group that keeps a row
+// in registers: a classifier's 1000 classes take a workgroup.
 template <bool H>
 void launch_softmax(hipStream_t st, const void* x, void* y, int rows, int n) {
-  const int g = n <= kSoftmaxRegs * 16 ? 16 : n <= kSoftmaxRegs * 64 ? 64 : 256;
-  auto* k = g == 16   ? softmax_rows_kernel<H, 16>
+  const int g = n <= 4 ? 1 : n <= 8 ? 2 : n <= 16 ? 4 : n <= kSoftmaxRegs * 16 ? 16 : n <= kSoftmaxRegs * 64 ? 64 : 256;
+  auto* k = g == 1    ? softmax_rows_kernel<H, 1>
+            : g == 2  ? softmax_rows_kernel<H, 2>
+            : g == 4  ? softmax_rows_kernel<H, 4>
+            : g == 16 ? softmax_rows_kernel<H, 16>
             : g == 64 ? softmax_rows_kernel<H, 64>
                       : softmax_rows_kernel<H, 256>;
   const long long blocks = ((long long)rows * g + 255) / 256;
