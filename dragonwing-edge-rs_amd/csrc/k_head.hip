@@ -135,6 +135,63 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_exact_kernel(const void* A,
   }
 }
 
+// The same sums with a thread per output straight from memory (j across the
+// lanes: B's rows coalesced, A's value the same in every lane).  The tiles
+// above cost about 2 us for 1024 workgroups before their first step; on many
+// outputs of few steps that is the whole product.
+template <bool F16, bool TB>
+__global__ __launch_bounds__(256) void gemm_thread_kernel(const void* A, const void* B, void* Cm, int m, int n, int k,
+                                                          const void* bias, int blen) {
+  using E = std::conditional_t<F16, uint16_t, float>;
+  const int j = blockIdx.x * 256 + threadIdx.x;
+  const int i = blockIdx.y;
+  if (j >= n || i >= m) return;
+  const E* a = (const E*)A + (size_t)i * k;
+  const E* b = (const E*)B + (TB ? (size_t)j * k : (size_t)j);
+  const size_t bs = TB ? 1 : (size_t)n;  // B's step along p
+  auto widen = [](E v) -> float {
+    if constexpr (F16) return h2f(v);
+    return v;
+  };
+  float acc = 0.0f;
+  for (int p = 0; p < k; ++p) {
+    const float x = widen(a[p]), y = widen(b[p * bs]);
+    if constexpr (TB) {
+      float prod = x * y;
+      asm("" : "+v"(prod));  // rounded product, then the add
+      acc = acc + prod;
+    } else {
+      acc = fmaf(x, y, acc);
+    }
+  }
+  if constexpr (F16) {
+    uint16_t hb = f2h(acc);
+    if (bias) hb = f16_add_bits(hb, ((const uint16_t*)bias)[j % blen]);
+    ((uint16_t*)Cm)[(size_t)i * n + j] = hb;
+  } else {
+    if (bias) acc = acc + ((const float*)bias)[j % blen];
+    ((float*)Cm)[(size_t)i * n + j] = acc;
+  }
+}
+
+// Whether a thread per output is expected to be done before the tiles, in
+// microseconds: its workgroups' dispatch, or a chain of K steps that the waves
+// in flight lengthen, against the tiles' workgroups.  Fitted to 9 shapes of up
+// to 6.5M outputs with K of 1 to 128, both kernels timed at each: 1024 x 1024
+// f32 with K = 8 4.4 against 17.9 us, with K = 64 14.9 against 20.6 us; 65535 x
+// 100 with K = 32 67 against 114 us; 32 x 1000 with K = 8 3.9 against 3.6 us,
+// with K = 128 13.8 against 3.8 us.  Above 64 steps it won nowhere by more
+// than 6%.
+bool gemm_by_threads(int dtype, bool trans_b, int m, int n, int k) {
+  if (k > 64) return false;
+  const float waves = (float)m * (float)((n - 1) / 64 + 1), blocks = (float)m * (float)((n - 1) / 256 + 1);
+  const float tiles = (float)((m - 1) / kGemmR + 1) * (float)((n - 1) / kGemmC + 1);
+  const float chain = 2.6f + (float)k * std::max(0.09f, (trans_b ? 1e-4f : 1.3e-5f) * waves);
+  const float t = std::max(std::max(3.8f, 0.00047f * blocks), chain);
+  const float per_tile = dtype == F32 ? (trans_b ? 0.0026f : 0.00172f) : (trans_b ? 0.003f : 0.00245f);
+  return t < std::max(3.6f, 2.3f + per_tile * tiles + 7e-6f * tiles * (float)k);
+}
+
 // int32 sum of i8 products (gemm_i8_scalar, ops.rs:2981-2995); integer
 // addition wraps like the reference's release build, in any order.
 __global__ __launch_bounds__(256) void gemm_i8_kernel(const int8_t* A, const int8_t* B, int32_t* Cm, int m, int n,
@@ -346,14 +403,22 @@ void launch_gemm_ex(hipStream_t st, int dtype, const void* a, const void* b, voi
   if (m > 65535) fail(-2, "gemm: more than 65535 rows");
   const long long cols = ((long long)n + kGemmC - 1) / kGemmC, gx = std::min(cols, kMaxGridX);
   const dim3 g((unsigned)gx, (unsigned)((m + kGemmR - 1) / kGemmR), (unsigned)((cols + gx - 1) / gx));
+  const bool threads = gemm_by_threads(dtype, trans_b, m, n, k);
+  const dim3 gt((unsigned)((n - 1) / 256 + 1), (unsigned)m);
+  auto launch = [&](auto* tile, auto* thread) {
+    if (threads)
+      hipLaunchKernelGGL(thread, gt, dim3(256), 0, st, a, b, c, m, n, k, bias, blen);
+    else
+      hipLaunchKernelGGL(tile, g, dim3(kGemmThreads), 0, st, a, b, c, m, n, k, bias, blen);
+  };
   if (dtype == F32 && !trans_b)
-    hipLaunchKernelGGL((gemm_exact_kernel<false, false>), g, dim3(kGemmThreads), 0, st, a, b, c, m, n, k, bias, blen);
+    launch(gemm_exact_kernel<false, false>, gemm_thread_kernel<false, false>);
   else if (dtype == F32)
-    hipLaunchKernelGGL((gemm_exact_kernel<false, true>), g, dim3(kGemmThreads), 0, st, a, b, c, m, n, k, bias, blen);
+    launch(gemm_exact_kernel<false, true>, gemm_thread_kernel<false, true>);
   else if (dtype == F16 && !trans_b)
-    hipLaunchKernelGGL((gemm_exact_kernel<true, false>), g, dim3(kGemmThreads), 0, st, a, b, c, m, n, k, bias, blen);
+    launch(gemm_exact_kernel<true, false>, gemm_thread_kernel<true, false>);
   else if (dtype == F16)
-    hipLaunchKernelGGL((gemm_exact_kernel<true, true>), g, dim3(kGemmThreads), 0, st, a, b, c, m, n, k, bias, blen);
+    launch(gemm_exact_kernel<true, true>, gemm_thread_kernel<true, true>);
   else
     fail(-2, "gemm: dtype");
   DW_HIP(hipGetLastError());

@@ -6,7 +6,9 @@ import time
 import numpy as np
 import pytest
 
+import oracle
 from dragonwing_edge_rs_amd import ops
+from dragonwing_edge_rs_amd.graph import GRAPH_F16, GRAPH_F32, Graph, HipGraphRuntime
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +43,41 @@ def test_softmax_of_short_rows(backend, rows, n):
     e = np.exp(x.astype(np.float64) - x.max(axis=1, keepdims=True))
     # the subtraction's half ulp of up to 20, exp's 2 ulps, at most 15 additions, two roundings
     np.testing.assert_allclose(got, e / e.sum(axis=1, keepdims=True), rtol=(20 / 2 + 2 + 15 + 2) * 2.0 ** -24)
+
+
+# in tiles of 256 steps of K, whatever K is: 3.5 to 5 times as long as the relu of as many values
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("m,n,k", [(1024, 1024, 8), (1, 100000, 3), (4097, 257, 5)])
+def test_gemm_of_few_steps(backend, m, n, k, f16):
+    r = np.random.default_rng(m + n + k)
+    a, b = r.normal(0, 1, (m, k)).astype(np.float32), r.normal(0, 0.2, (k, n)).astype(np.float32)
+    f, want = ops.gemm_f32, oracle.gemm_f32
+    if f16:
+        a, b = a.astype(np.float16).view(np.uint16), b.astype(np.float16).view(np.uint16)
+        f, want = ops.gemm_fp16, oracle.gemm_fp16
+    ba, bb, bc = backend.from_numpy(a), backend.from_numpy(b), backend.alloc(m * n * a.itemsize)
+    t = per_call(backend, lambda: f(backend, ba, bb, bc, m, n, k))
+    assert t < 2.5 * relu_time(backend, m * n)
+    np.testing.assert_array_equal(backend.to_numpy(bc, a.dtype, (m, n)), want(a, b))
+
+
+@pytest.mark.parametrize("f16", [False, True])
+def test_transposed_gemm_of_few_steps(backend, f16):
+    from oracle.cpu_graph import CpuGraph
+    m, n, k = 1500, 700, 4
+    r = np.random.default_rng(k + f16)
+    dt, cast = ("f16", lambda v: v.astype(np.float16).view(np.uint16)) if f16 else ("f32", lambda v: v.astype(np.float32))
+    x, w, b = cast(r.normal(0, 1, (m, k))), cast(r.normal(0, 0.2, (n, k))), cast(r.normal(0, 1, n))
+    g = Graph(GRAPH_F16 if f16 else GRAPH_F32)
+    g.add_tensor("x", x.shape, dt)
+    g.add_initializer("w", w, dt)
+    g.add_initializer("b", b, dt)
+    g.add_tensor("y", (m, n), dt)
+    g.add_op("fc", "Gemm", ["x", "w", "b"], ["y"], trans_b=1)
+    g.set_io(["x"], ["y"])
+    rt = HipGraphRuntime(g, backend)
+    rt.set_input_bytes("x", x)
+    assert per_call(backend, rt.run) < 3 * relu_time(backend, m * n)
+    cg = CpuGraph(g.to_dict(), g.initializer)
+    cg.set_input("x", x)
+    np.testing.assert_array_equal(rt.get_output_bytes("y").view(x.dtype).reshape(m, n), cg.run()["y"])
