@@ -248,7 +248,11 @@ __device__ __forceinline__ void store_outputs(const DirectArgs& a, const float* 
 // The 1x1 exact-order kernel (k_direct1x1.hip); false if the problem is not
 // one it handles.
 bool launch_conv1x1_exact(hipStream_t st, const DirectArgs& a);
-// f32 in and out, any shape (k_conv_f32.hip); false if its 32-bit offsets do not reach
-bool launch_conv_f32(hipStream_t st, const DirectArgs& a);
+// the channels that one of its waves takes; 0 if the problem is not one it handles
+int conv1x1_exact_channels(const DirectArgs& a);
+// The register-tiled kernel, f32 in and out, any shape (k_conv_f32.hip).
+bool conv_f32_reaches(const DirectArgs& a);  // its 32-bit offsets do
+float conv_f32_cost(const DirectArgs& a);    // expected microseconds, of layers of few channels
+void launch_conv_f32(hipStream_t st, const DirectArgs& a);
 
 }  // namespace dw

@@ -292,6 +292,8 @@ void launch_direct_conv(hipStream_t st, const DirectArgs& a);
 bool stem_pad_ok(const DirectArgs& a);
 // true if a runs on the f32 window kernel once its weights are packed (wq)
 bool conv_window_f32_ok(const DirectArgs& a);
+// true if a runs on the register-tiled f32 kernel (unless the window kernel or the stem's takes it)
+bool conv_f32_tiles(const DirectArgs& a);
 bool conv1x1_u8_f16_supported(int cin, int cout);
 void launch_strided_copy(hipStream_t st, const StridedCopyArgs& a);
 void launch_broadcast_binary(hipStream_t st, const BinaryArgs& a);

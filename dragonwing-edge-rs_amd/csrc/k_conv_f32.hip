@@ -253,17 +253,71 @@ void launch_tile(hipStream_t st, CfArgs a) {
   DW_HIP(hipGetLastError());
 }
 
+// The tile that is expected to be done first, in microseconds: what a
+// workgroup's chunks and FMAs cost alone, and what the busiest CU's
+// workgroups cost its FMAs, LDS reads and barriers.  The coefficients are a
+// non-negative least squares fit (14%) to 12 tiles on 33 convolutions of
+// 180 to 205k pixels, 3-256 input and 16-256 output channels; the choice
+// is 5% off the best tile (geometric mean).  A chunk of K that is a few
+// hundred nanoseconds of latency whatever it holds asks for small tiles
+// and long chunks on few pixels (20 x 20, 128 -> 128: 18.5 us at 1 x 1
+// against 46.7 us at 2 x 4, with a repacking launch that is gone), FMAs per LDS read for large ones on many (16
+// x 80 x 80, 64 -> 64: 140 us at 4 x 4 against 243 us at 1 x 2).
+struct CfChoice {
+  int px, ch;
+  long long wgs;
+};
+CfChoice cf_choose(const DirectArgs& d) {
+  CfChoice best{};
+  float least = 0;
+  const int taps = d.kh * d.kw;
+  const float kt = (float)taps * (float)d.cin / 64.0f;
+  for (int p : {1, 2, 4})
+    for (int c : {1, 2, 3, 4, 5}) {
+      if (c == 1 && p > 1) continue;
+      const long long wgs = (((long long)d.m + 32 * p - 1) / (32 * p)) * ((d.cout + 8 * c - 1) / (8 * c));
+      const float mean = (float)wgs / 256.0f, full = (float)((wgs + 255) / 256);
+      const float chunks = (float)cf_chunks(d.cin, taps, p), fmas = kt * (float)(p * c);
+      const float cost = 0.448f * chunks + 0.103f * fmas +
+                         full * (0.0779f * fmas + 0.0043f * kt * (float)(p + c) + 0.242f * chunks) + 0.682f * mean;
+      if (!best.px || cost < least) {
+        least = cost;
+        best = {p, c, wgs};
+      }
+    }
+  return best;
+}
+
 }  // namespace
 
-bool launch_conv_f32(hipStream_t st, const DirectArgs& d) {
+bool conv_f32_reaches(const DirectArgs& d) {
   // 32-bit byte offsets into the input and the weights, also for the windows
   // and chunks that reach past them
-  if (d.in_kind != 0 || d.out_kind != 0 || d.m <= 0) return false;
   const long long xe = ((long long)d.n * d.h * d.w - 1) * d.x_pix_stride + d.cin;
   const long long we = (long long)d.kh * d.kw * d.cin * d.cout;
   const long long edge = ((long long)(d.pt + d.kh + 64) * d.w + d.pl + d.kw) * d.x_pix_stride + 64;
   const long long wedge = (64ll * d.cin + 64) * d.cout + d.cout;
-  if (xe + edge >= (1ll << 29) || we + wedge >= (1ll << 29)) return false;
+  return d.m > 0 && d.cout <= 8 * 65535 && xe + edge < (1ll << 29) && we + wedge < (1ll << 29);
+}
+
+// The same kind of sum for layers of up to 24 input or 4 output channels,
+// where the tile's per-tap work (a tap is a segment of few steps, kept and put
+// back at the borders) and its eight channels a row of threads weigh: a
+// robust fit (15%) to 627 of them.
+float conv_f32_cost(const DirectArgs& d) {
+  const CfChoice t = cf_choose(d);
+  const int taps = d.kh * d.kw;
+  const float chunks = (float)cf_chunks(d.cin, taps, t.px), segs = cf_taps(d.cin, taps, t.px) ? (float)taps : chunks;
+  const float kt = (float)taps * (float)d.cin / 64.0f, pc = (float)(t.px * t.ch);
+  const float mean = (float)t.wgs / 256.0f, full = (float)((t.wgs + 255) / 256);
+  return 3.26f + 0.673f * chunks + 0.0476f * segs + 0.0542f * kt * pc +
+         full * (0.0782f * segs + 0.108f * kt * (float)(t.px + t.ch) + 0.0398f * kt * pc) + 0.139f * mean * pc;
+}
+
+void launch_conv_f32(hipStream_t st, const DirectArgs& d) {
+  if (d.in_kind != 0 || d.out_kind != 0 || !conv_f32_reaches(d)) fail(-4, "conv_f32: not a problem of this kernel");
+  const long long xe = ((long long)d.n * d.h * d.w - 1) * d.x_pix_stride + d.cin;
+  const long long we = (long long)d.kh * d.kw * d.cin * d.cout;
   CfArgs a{};
   a.x = (const float*)d.x + d.x_c_off;
   a.w = d.wf;
@@ -276,35 +330,7 @@ bool launch_conv_f32(hipStream_t st, const DirectArgs& d) {
   a.act = d.act;
   a.x_bytes = (int)(xe * 4);
   a.w_bytes = (int)(we * 4);
-  // The tile that is expected to be done first, in microseconds: what a
-  // workgroup's chunks and FMAs cost alone, and what the busiest CU's
-  // workgroups cost its FMAs, LDS reads and barriers.  The coefficients are a
-  // non-negative least squares fit (14%) to 12 tiles on 33 convolutions of
-  // 180 to 205k pixels, 3-256 input and 16-256 output channels; the choice
-  // is 5% off the best tile (geometric mean).  A chunk of K that is a few
-  // hundred nanoseconds of latency whatever it holds asks for small tiles
-  // and long chunks on few pixels (20 x 20, 128 -> 128: 18.5 us at 1 x 1
-  // against 46.7 us at 2 x 4, with a repacking launch that is gone), FMAs per LDS read for large ones on many (16
-  // x 80 x 80, 64 -> 64: 140 us at 4 x 4 against 243 us at 1 x 2).
-  float least = 0;
-  int px = 0, ch = 0;
-  const int taps = d.kh * d.kw;
-  const float kt = (float)taps * (float)d.cin / 64.0f;
-  for (int p : {1, 2, 4})
-    for (int c : {1, 2, 3, 4, 5}) {
-      if (c == 1 && p > 1) continue;
-      const long long wgs = (((long long)d.m + 32 * p - 1) / (32 * p)) * ((d.cout + 8 * c - 1) / (8 * c));
-      const float mean = (float)wgs / 256.0f, full = (float)((wgs + 255) / 256);
-      const float chunks = (float)cf_chunks(d.cin, taps, p), fmas = kt * (float)(p * c);
-      const float cost = 0.448f * chunks + 0.103f * fmas +
-                         full * (0.0779f * fmas + 0.0043f * kt * (float)(p + c) + 0.242f * chunks) + 0.682f * mean;
-      if (!px || cost < least) {
-        least = cost;
-        px = p;
-        ch = c;
-      }
-    }
-  if ((d.cout + 8 * ch - 1) / (8 * ch) > 65535) return false;
+  const auto [px, ch, wgs] = cf_choose(d);
   const bool vec = d.cin % 4 == 0 && d.x_pix_stride % 4 == 0 && (uintptr_t)a.x % 16 == 0;
 #define DW_CF(P, C) \
   if (px == P && ch == C) vec ? launch_tile<P, C, true>(st, a) : launch_tile<P, C, false>(st, a);
@@ -312,7 +338,6 @@ bool launch_conv_f32(hipStream_t st, const DirectArgs& d) {
   DW_CF(2, 2) DW_CF(2, 3) DW_CF(2, 4) DW_CF(2, 5)
   DW_CF(4, 2) DW_CF(4, 3) DW_CF(4, 4) DW_CF(4, 5)
 #undef DW_CF
-  return true;
 }
 
 }  // namespace dw

@@ -9,8 +9,8 @@
 // for (tap, ic) is wave-uniform and is fetched with scalar loads, and each
 // input value is read and decoded once for the whole chunk.  Used for
 // convolutions whose c_in is not a multiple of 8 (the
-// 3-channel stem), and for the fp16 layers of the int8 graph that must match
-// the CPU bit for bit.
+// 3-channel stem), for the fp16 layers of the int8 graph that must match
+// the CPU bit for bit, and for fp32 layers of few channels.
 //
 // dwconv: depthwise of any k and stride, channel multiplier 1 (3x3 at stride 1
 // or 2 is dwconv3_kernel's, k_dwconv3.hip).  One thread = one
@@ -622,14 +622,16 @@ bool stem_pad_ok(const DirectArgs& a) {
 // tile in LDS, weights packed by channel quads) reads each input once and
 // starts with everything in flight, which suits a layer of at most a wave per
 // SIMD: 1 x 56 x 56 x 64 -> 64 takes 14.2 us with the packing, against 17-19
-// us on conv_f32_kernel; on 4 x 40 x 40 it is 34.5 against 22 us.
+// us on conv_f32_kernel; on 4 x 40 x 40 it is 34.5 against 22 us.  Of 4 output
+// channels the other kernel's tile wastes half: 95k pixels of 32 -> 4 17.3
+// against 30.6 us.  And it takes what lies past the other's 32-bit offsets.
 bool conv_window_f32_ok(const DirectArgs& a) {
   constexpr int TH = 16, TW = 16;
   if (a.in_kind != 0 || !(a.cin == 32 || a.cin == 64) || a.cout % 4 != 0 || a.kh * a.kw * a.cin > kTileWRows ||
       (a.kh == 1 && a.kw == 1) || (a.x_pix_stride * 4) % 16 != 0 || (a.x_c_off * 4) % 16 != 0 ||
       ((uintptr_t)a.x & 15) != 0)
     return false;
-  if (((long long)a.m + 63) / 64 * (a.cout / 4) > 1024) return false;
+  if (((long long)a.m + 63) / 64 * (a.cout / 4) > 1024 && a.cout > 4 && conv_f32_reaches(a)) return false;
   // the window's channel quads in at most 24 loads per thread
   const int iwin_w = (TW - 1) * a.sw + a.kw, iwin_h = (TH - 1) * a.sh + a.kh;
   const long long xbytes = (((long long)a.n * a.h * a.w - 1) * a.x_pix_stride + a.x_c_off + a.cin) * 4;
@@ -637,8 +639,58 @@ bool conv_window_f32_ok(const DirectArgs& a) {
          iwin_w <= 2 * (TH * TW / (a.cin / 4)) && xbytes < (1ll << 31);
 }
 
+namespace {
+// 16-byte input vectors: c_in a whole number of them, on aligned addresses.
+bool vec_in(const DirectArgs& a) {
+  const int es = a.in_kind == 0 ? 4 : (a.in_kind == 1 ? 2 : 1);
+  return a.cin % (16 / es) == 0 && (a.x_pix_stride * es) % 16 == 0 && (a.x_c_off * es) % 16 == 0 &&
+         ((uintptr_t)a.x & 15) == 0;
+}
+
+// Output channels per thread of direct_conv_kernel: the widest chunk of c_out
+// that still gives about four wavefronts per CU (wide chunks pay the input
+// decode once for more FMAs; narrow ones spread small layers over the GPU).
+int direct_channels(const DirectArgs& a, bool vin) {
+  const long waves = ((long)a.m + 63) / 64;
+  static const int wide[] = {80, 64, 40, 32, 16, 8, 4, 1};
+  static const int narrow[] = {16, 8, 4, 1};
+  const int* cand = vin ? wide : narrow;
+  const int ncand = vin ? 8 : 4;
+  // (chunks below 4 channels only when c_out is not a multiple of 4)
+  const int min_oc = a.cout % 4 == 0 ? 4 : 1;
+  for (int i = 0; i < ncand; ++i)
+    if (cand[i] >= min_oc && a.cout % cand[i] == 0 && waves * (a.cout / cand[i]) >= 1024) return cand[i];
+  return min_oc;  // too few pixels for any chunk: the narrowest
+}
+}  // namespace
+
+// fp32 layers run on conv_f32_kernel unless they have few channels (it pays a
+// chunk and a segment per tap, and whole rows of 8 channels: 640 x 640, 4 -> 1
+// 1x1 19.4 us against 4.4 us, 32 x 112 x 112, 3 -> 8 7x7/2 72.7 against 22.5
+// us) and this file's or the 1x1 kernel is expected to be done first.  Both
+// costs are robust fits (17-40% and 15%) to 627 layers timed on both sides,
+// with up to 24 input or 4 output channels; the tiles have to be 20% ahead,
+// and are then slower than the other kernel on 1% of them.  Of 242 layers of
+// more channels the tiles were never slower but on 1-4 output channels.
+bool conv_f32_tiles(const DirectArgs& a) {
+  if (a.in_kind != 0 || a.out_kind != 0 || !conv_f32_reaches(a)) return false;
+  if (a.cin > 24 && a.cout > 4) return true;
+  const float taps = (float)(a.kh * a.kw), K = taps * (float)a.cin;
+  const bool vin = vec_in(a);
+  const int c1 = conv1x1_exact_channels(a), c = c1 ? c1 : direct_channels(a, vin);
+  const long waves = ((long)a.m + 63) / 64 * (a.cout / c);
+  const float g = (float)waves / 1024.0f, full = (float)((waves + 1023) / 1024), o = (float)c;
+  const float direct = c1    ? 3.78f + full * (0.4f + K * (0.00796f + 0.00432f * o)) + 0.0466f * g * o
+                       : vin ? 3.21f + 0.0267f * taps + 0.00371f * K * o + 0.0281f * full * K + 0.135f * g * o +
+                                   0.000245f * g * K * o
+                             : 3.61f + 0.0253f * taps + K * (0.0336f + 0.00249f * o) + 0.0406f * full * K +
+                                   0.132f * g * o;
+  return direct >= 1.2f * conv_f32_cost(a);
+}
+
 void launch_direct_conv(hipStream_t st, const DirectArgs& a_in) {
-  if (launch_conv1x1_exact(st, a_in)) return;
+  const bool tiles = conv_f32_tiles(a_in);
+  if (!tiles && launch_conv1x1_exact(st, a_in)) return;
   DirectArgs a = a_in;
   // the 3x3, 3-channel stem
   if (a.in_kind == 3 && !(a.kh == 3 && a.kw == 3 && a.cin == 3 && a.cout % 16 == 0))
@@ -694,10 +746,6 @@ void launch_direct_conv(hipStream_t st, const DirectArgs& a_in) {
     DW_HIP(hipGetLastError());
     return;
   }
-  const int es = a.in_kind == 0 ? 4 : (a.in_kind == 1 ? 2 : 1);
-  const int vn = 16 / es;
-  const bool vin = a.cin % vn == 0 && (a.x_pix_stride * es) % 16 == 0 && (a.x_c_off * es) % 16 == 0 &&
-                   ((uintptr_t)a.x & 15) == 0;
   if (a.wq && conv_window_f32_ok(a)) {
     constexpr int TH = 16, TW = 16, C = 4;
     const int iwin_w = (TW - 1) * a.sw + a.kw;
@@ -719,22 +767,9 @@ void launch_direct_conv(hipStream_t st, const DirectArgs& a_in) {
     DW_HIP(hipGetLastError());
     return;
   }
-  if (launch_conv_f32(st, a)) return;
-  // Output channels per thread: the widest chunk of c_out that still gives
-  // about four wavefronts per CU (wide chunks pay the input decode once for
-  // more FMAs; narrow ones spread small layers over the GPU).
-  const long waves = ((long)a.m + 63) / 64;
-  static const int wide[] = {80, 64, 40, 32, 16, 8, 4, 1};
-  static const int narrow[] = {16, 8, 4, 1};
-  // (f32 comes here only past conv_f32_kernel's 32-bit offsets)
-  const int* cand = a.in_kind == 0 ? narrow + 2 : vin ? wide : narrow;
-  const int ncand = a.in_kind == 0 ? 2 : vin ? 8 : 4;
-  // (chunks below 4 channels only when c_out is not a multiple of 4)
-  const int min_oc = a.cout % 4 == 0 ? 4 : 1;
-  int oc = 0;
-  for (int i = 0; i < ncand && !oc; ++i)
-    if (cand[i] >= min_oc && a.cout % cand[i] == 0 && waves * (a.cout / cand[i]) >= 1024) oc = cand[i];
-  if (!oc) oc = min_oc;  // too few pixels for any chunk: the narrowest
+  if (tiles) return launch_conv_f32(st, a);
+  const bool vin = vec_in(a);
+  const int oc = direct_channels(a, vin);
   if (a.cout % oc != 0) fail(-2, "direct conv: no channel chunk for this c_out");
   const int oes = a.out_kind == 0 ? 4 : (a.out_kind == 1 ? 2 : 1);
   auto aligned = [&](int v) {
@@ -749,11 +784,7 @@ void launch_direct_conv(hipStream_t st, const DirectArgs& a_in) {
     DW_HIP(hipGetLastError());                                                                \
     return;                                                                                   \
   }
-#define DW_DC_ALL(O, V) DW_DC(1, O, V) DW_DC(2, O, V)
-  DW_DC(0, 4, true)
-  DW_DC(0, 1, true)
-  DW_DC(0, 4, false)
-  DW_DC(0, 1, false)
+#define DW_DC_ALL(O, V) DW_DC(0, O, V) DW_DC(1, O, V) DW_DC(2, O, V)
   DW_DC_ALL(80, true)
   DW_DC_ALL(64, true)
   DW_DC_ALL(40, true)

@@ -140,35 +140,40 @@ __global__ __launch_bounds__(64) void conv1x1_exact_kernel(const DirectArgs a) {
 
 }  // namespace
 
-bool launch_conv1x1_exact(hipStream_t st, const DirectArgs& a_in) {
-  if (a_in.in_kind == 0 || a_in.kh != 1 || a_in.kw != 1 || a_in.pt != 0 || a_in.pl != 0) return false;
-  const int es = a_in.in_kind == 1 ? 2 : 1;
+// Channels per wave C and pixels per lane P.  Measured on the detect-head
+// shapes (u8 -> f16, 64 and 80 channels, 40x40 to 80x80, batch 32), one
+// pixel per lane with 16 channels is fastest: the wave keeps few
+// registers, so many waves per SIMD hide the scalar weight loads and the
+// input loads, and each decoded input still feeds 16 FMAs.  Narrower
+// groups are used when c_out needs them or the layer has too few pixels
+// for one wave per SIMD.  The grid runs all pixel tiles of one channel
+// group before the next, so the waves in flight share one group's weights
+// in the scalar cache.
+int conv1x1_exact_channels(const DirectArgs& a) {
+  if (a.kh != 1 || a.kw != 1 || a.pt != 0 || a.pl != 0) return 0;
+  const int es = a.in_kind == 0 ? 4 : (a.in_kind == 1 ? 2 : 1);
   const int vn = 16 / es;
-  if (a_in.cin % vn != 0 || (a_in.x_pix_stride * es) % 16 != 0 || (a_in.x_c_off * es) % 16 != 0 ||
-      ((uintptr_t)a_in.x & 15) != 0)
-    return false;
-  // Channels per wave C and pixels per lane P.  Measured on the detect-head
-  // shapes (u8 -> f16, 64 and 80 channels, 40x40 to 80x80, batch 32), one
-  // pixel per lane with 16 channels is fastest: the wave keeps few
-  // registers, so many waves per SIMD hide the scalar weight loads and the
-  // input loads, and each decoded input still feeds 16 FMAs.  Narrower
-  // groups are used when c_out needs them or the layer has too few pixels
-  // for one wave per SIMD.  The grid runs all pixel tiles of one channel
-  // group before the next, so the waves in flight share one group's weights
-  // in the scalar cache.
+  if (a.cin % vn != 0 || (a.x_pix_stride * es) % 16 != 0 || (a.x_c_off * es) % 16 != 0 || ((uintptr_t)a.x & 15) != 0)
+    return 0;
+  int best = 0;
+  for (int c : {16, 8, 4})
+    if (a.cout % c == 0) {
+      best = c;
+      const long waves = (long)((a.m + 63) / 64) * (a.cout / c);
+      if (waves >= 1024) break;
+    }
+  return best;
+}
+
+bool launch_conv1x1_exact(hipStream_t st, const DirectArgs& a_in) {
   struct Opt {
     int c, p;
   };
   static const Opt opts[] = {{20, 4}, {16, 4}, {40, 2}, {32, 2}, {8, 4}, {40, 1}, {20, 1}, {16, 1},
                              {4, 4},  {8, 1},  {4, 1}};
+  Opt best{conv1x1_exact_channels(a_in), 1};
+  if (!best.c) return false;
   const bool nosub = a_in.in_kind == 2 && fabsf(a_in.in_scale) >= 6.103515625e-05f;
-  Opt best{0, 0};
-  for (int c : {16, 8, 4})
-    if (a_in.cout % c == 0) {
-      best = {c, 1};
-      const long waves = (long)((a_in.m + 63) / 64) * (a_in.cout / c);
-      if (waves >= 1024) break;
-    }
   // Override for tests and tuning runs: "C,P", applied where valid.
   if (const char* env = getenv("DW_DIRECT1X1")) {
     int c = 0, pp = 0;
@@ -176,7 +181,6 @@ bool launch_conv1x1_exact(hipStream_t st, const DirectArgs& a_in) {
       for (const Opt& o : opts)
         if (o.c == c && o.p == pp && a_in.cout % c == 0) best = o;
   }
-  if (!best.c) return false;
   DirectArgs a = a_in;
   const int oes = a.out_kind == 0 ? 4 : (a.out_kind == 1 ? 2 : 1);
   auto aligned = [&](int v) {
@@ -195,7 +199,7 @@ bool launch_conv1x1_exact(hipStream_t st, const DirectArgs& a_in) {
     DW_HIP(hipGetLastError());                                                                      \
     return true;                                                                                    \
   }
-#define DW_K_ALL(CC, PP) DW_K(1, CC, PP, false) DW_K(2, CC, PP, false) DW_K(2, CC, PP, true)
+#define DW_K_ALL(CC, PP) DW_K(0, CC, PP, false) DW_K(1, CC, PP, false) DW_K(2, CC, PP, false) DW_K(2, CC, PP, true)
   DW_K_ALL(20, 4)
   DW_K_ALL(16, 4)
   DW_K_ALL(40, 2)

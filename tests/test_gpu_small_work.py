@@ -81,3 +81,61 @@ def test_transposed_gemm_of_few_steps(backend, f16):
     cg = CpuGraph(g.to_dict(), g.initializer)
     cg.set_input("x", x)
     np.testing.assert_array_equal(rt.get_output_bytes("y").view(x.dtype).reshape(m, n), cg.run()["y"])
+
+
+def conv_f32(backend, bx, bw, by, x_shape, w_shape, s, p):
+    n, h, w, ci = x_shape
+    ops.conv2d_bias_act_f32_nhwc(backend, bx, bw, None, by, n, h, w, ci, w_shape[3], *w_shape[:2], s, s, p, p)
+
+
+# on the register-tiled kernel: 4 to 13 times as long as the relu of the input (19 times with 7 x 7 taps)
+@pytest.mark.parametrize("x_shape,w_shape,s,limit", [
+    ((1, 640, 641, 4), (1, 1, 4, 1), 1, 2),
+    ((1, 640, 639, 1), (3, 3, 1, 1), 1, 3),
+    ((32, 112, 111, 3), (7, 7, 3, 8), 2, 9),
+    ((8, 150, 151, 5), (1, 1, 5, 11), 1, 3),
+])
+def test_conv_f32_of_few_channels(backend, x_shape, w_shape, s, limit):
+    r = np.random.default_rng(x_shape[2])
+    x, w = r.uniform(-1, 1, x_shape).astype(np.float32), r.uniform(-1, 1, w_shape).astype(np.float32)
+    p = w_shape[0] // 2
+    want = oracle.conv2d_f32_nhwc(x, w, (s, s), (p, p))
+    bx, bw, by = backend.from_numpy(x), backend.from_numpy(w), backend.alloc(want.nbytes)
+    t = per_call(backend, lambda: conv_f32(backend, bx, bw, by, x_shape, w_shape, s, p))
+    np.testing.assert_array_equal(backend.to_numpy(by, np.float32, want.shape), want)
+    assert t < limit * relu_time(backend, max(x.size, want.size))
+
+
+@pytest.mark.parametrize("x_shape,w_shape", [
+    # few channels on the side of the rule that keeps the tiles: odd quads of K and several taps a chunk
+    ((1, 20, 21, 13), (5, 5, 13, 17)), ((2, 31, 33, 3), (7, 7, 3, 101)), ((4, 40, 41, 7), (3, 3, 7, 70)),
+    ((1, 14, 15, 11), (3, 3, 11, 45)), ((1, 5, 6, 24), (5, 5, 24, 3)), ((1, 20, 20, 65), (3, 3, 65, 2)),
+    # on the other: one channel, a 1x1 on 4, many channels from one, the window kernel's 4 output channels
+    ((1, 40, 41, 1), (3, 3, 1, 1)), ((2, 33, 34, 4), (1, 1, 4, 24)), ((2, 25, 26, 1), (7, 7, 1, 97)),
+    ((4, 90, 91, 48), (3, 3, 48, 1)), ((9, 101, 102, 32), (3, 3, 32, 4)),
+])
+def test_conv_f32_on_both_sides_of_the_rule(backend, x_shape, w_shape):
+    r = np.random.default_rng(x_shape[1])
+    x, w = r.uniform(-1, 1, x_shape).astype(np.float32), r.uniform(-1, 1, w_shape).astype(np.float32)
+    p = w_shape[0] // 2
+    want = oracle.conv2d_f32_nhwc(x, w, (1, 1), (p, p))
+    by = backend.alloc(want.nbytes)
+    conv_f32(backend, backend.from_numpy(x), backend.from_numpy(w), by, x_shape, w_shape, 1, p)
+    np.testing.assert_array_equal(backend.to_numpy(by, np.float32, want.shape), want)
+
+
+def test_conv_f32_past_the_tiles_offsets(backend):
+    # 2 GB of input, past the register tiles' 32-bit offsets: 3 times as long as half of it, which they reach
+    # (11 times with 4 channels a thread)
+    w_shape, times = (1, 1, 64, 16), []
+    r = np.random.default_rng(2)
+    block = r.uniform(-1, 1, (1, 5, 16384, 64)).astype(np.float32)
+    w = r.uniform(-1, 1, w_shape).astype(np.float32)
+    bw = backend.from_numpy(w)
+    for h in (255, 510):
+        shape = (1, h, 16384, 64)
+        bx, by = backend.from_numpy(np.resize(block, shape)), backend.alloc(h * 16384 * 16 * 4)
+        times.append(per_call(backend, lambda: conv_f32(backend, bx, bw, by, shape, w_shape, 1, 0), calls=3))
+        got = backend.to_numpy(by, np.float32, (h // 5, 5, 16384, 16))
+        np.testing.assert_array_equal(got, np.broadcast_to(oracle.conv2d_f32_nhwc(block, w, (1, 1), (0, 0)), got.shape))
+    assert times[1] < 6 * times[0]
