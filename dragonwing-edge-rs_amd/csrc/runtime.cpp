@@ -1937,7 +1937,8 @@ void Runtime::emit_conv(const Group& gr) {
       for (size_t i = 0; i < W.numel() && fin; ++i) fin = (((const uint16_t*)W.data.data())[i] & 0x7c00) != 0x7c00;
     a.w_finite = fin ? 1 : 0;
   }
-  if (kh == 1 && kw == 1 && co % 16 == 0 && (W.dtype == DW_DTYPE_F32 || W.dtype == DW_DTYPE_F16)) {
+  if (kh == 1 && kw == 1 && co % 16 == 0 && (W.dtype == DW_DTYPE_F32 || W.dtype == DW_DTYPE_F16) &&
+      !conv_f32_tiles(a)) {
     // the 1x1 kernel's layout: [co / 16][ci][16] (each 16-channel group's
     // weight rows contiguous)
     std::vector<float> w(W.numel());
@@ -1951,8 +1952,8 @@ void Runtime::emit_conv(const Group& gr) {
         for (int j = 0; j < 16; ++j) wq[((size_t)g16 * ci + r) * 16 + j] = w[(size_t)r * co + 16 * g16 + j];
     a.wq16 = (const float*)upload(wq.data(), wq.size() * 4);
   }
-  if (a.in_kind == 0 && W.dtype == DW_DTYPE_F32 && ci % 16 == 0 && co % 4 == 0) {
-    // the tiled kernel's layout: [co / 4][kh * kw * ci][4]
+  if (W.dtype == DW_DTYPE_F32 && conv_window_f32_ok(a)) {
+    // the window kernel's layout: [co / 4][kh * kw * ci][4]
     const size_t rows = (size_t)kh * kw * ci;
     std::vector<float> wq(wf.size());
     for (int g4 = 0; g4 < co / 4; ++g4)
