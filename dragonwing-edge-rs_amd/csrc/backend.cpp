@@ -358,6 +358,7 @@ int dw_hip_download(dw_hip_backend* be, const dw_hip_buffer* src, void* dst, siz
   if (len != src->len)
     dw::fail(DW_ERR_INVALID, "download size mismatch: buffer " + std::to_string(src->len) +
                                  " bytes, destination " + std::to_string(len) + " bytes");
+  if (len && !dst) dw::fail(DW_ERR_INVALID, "null destination");
   b->download(dst, src->ptr, len);
   API_END
 }

@@ -3201,6 +3201,7 @@ int dw_hip_graph_get_output_f32(dw_hip_graph_runtime* rth, const char* name, flo
   const dw::RtTensor& t = output_tensor(rt, name);
   const size_t n = (size_t)(t.pixels() * t.c);
   if (count != n) dw::fail(DW_ERR_RUNTIME, "output size mismatch");
+  if (n && !data) dw::fail(DW_ERR_INVALID, "null data");
   if (t.dtype != dw::F32 && t.dtype != dw::F16 && t.dtype != dw::U8)
     dw::fail(DW_ERR_RUNTIME, "unsupported dtype for get_output_f32");
   if (t.dtype == dw::F32) {

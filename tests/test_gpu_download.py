@@ -4,11 +4,13 @@ device's."""
 import numpy as np
 import pytest
 
+from dragonwing_edge_rs_amd._lib import HipError, check, load
 from dragonwing_edge_rs_amd.graph import GRAPH_F16, GRAPH_F32, Graph, HipGraphRuntime
 
 pytestmark = pytest.mark.gpu
 
 MIB = 1 << 20
+DW_ERR_INVALID = -4
 
 
 @pytest.mark.parametrize("n", [1, 4095, 131073, MIB, MIB + 1, 4 * MIB - 1, 4 * MIB, 9 * MIB + 77,
@@ -49,3 +51,23 @@ def test_sliced_tensors(backend, dtype, pixels):
         for name, w in zip(("r0", "r1", "y"), want):
             np.testing.assert_array_equal(rt.get_output_bytes(name).view(np_t).reshape(w.shape), w)
             np.testing.assert_array_equal(rt.get_output_f32(name, w.size).reshape(w.shape), w.astype(np.float32))
+
+
+def test_null_destinations_are_refused(backend):
+    buf = backend.alloc(24)
+    with pytest.raises(HipError, match="null") as e:
+        check(load().dw_hip_download(backend.handle, buf.handle, None, 24))
+    assert e.value.code == DW_ERR_INVALID
+    g = Graph(GRAPH_F32)
+    for name in ("x", "y"):
+        g.add_tensor(name, (1, 2, 1, 3))
+    g.add_op("relu", "Relu", ["x"], ["y"])
+    g.set_io(["x"], ["y"])
+    rt = HipGraphRuntime(g, backend)
+    rt.set_input_f32("x", np.ones(6, np.float32))
+    rt.run()
+    for f, size in ((load().dw_hip_graph_get_output_f32, 6), (load().dw_hip_graph_get_output_bytes, 24)):
+        with pytest.raises(HipError, match="null") as e:
+            check(f(rt._h, b"y", None, size))
+        assert e.value.code == DW_ERR_INVALID
+    np.testing.assert_array_equal(rt.get_output_f32("y", 6), 1)
