@@ -88,8 +88,11 @@ hipError_t Backend::copy_chunks(uint8_t* dst, const uint8_t* src, size_t bytes, 
 // Through the page-locked slots: HIP's own copy to ordinary memory
 // runs at 18 GB/s, and one to page-locked memory at 56 GB/s of which a thread
 // moves 31 GB/s on (less into pages touched for the first time), so from 4 MiB
-// on four threads copy.  Measured into warm memory: 0.46 MB 37 us, 1.8 MB 90
-// us, 59 MB 1.56 ms (38 GB/s).
+// on four threads copy.  Measured into warm memory: 1.8 MB 85 us, 59 MB 1.56
+// ms (38 GB/s).  Up to 1 MiB a kernel fills the slot, whose end is the only
+// thing waited for: 64 KiB 12.8 us, 1 MiB 58 us.  HIP's copies of more than 16
+// KiB take 6 us longer there, or 110 us (seen after a 2 GB allocation was
+// freed), and those to ordinary memory 12.5 and 60 us, or 130 and 145.
 void Backend::download(void* dst, const void* src, size_t bytes) {
   hipPointerAttribute_t at{};
   if (bytes && hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered) {
@@ -104,12 +107,16 @@ void Backend::download(void* dst, const void* src, size_t bytes) {
     }
     uint8_t* d = (uint8_t*)dst;
     const uint8_t* s = (const uint8_t*)src;
+    const size_t mib = (size_t)1 << 20;
+    if (bytes <= mib) {
+      launch_copy(stream, s, slots, (unsigned)bytes, slot_ev[0]);
+      DW_HIP(hipEventSynchronize(slot_ev[0]));
+      memcpy(d, slots, bytes);
+      return;
+    }
     // a chunk costs about 10 us beside its bytes, which half a MiB hides; large
     // downloads take whole slots
-    const size_t mib = (size_t)1 << 20;
-    const size_t chunk = bytes >= 16 * mib ? kSlotBytes
-                         : bytes <= mib    ? bytes
-                                           : std::min(mib, (bytes / 2 + 4095) & ~(size_t)4095);
+    const size_t chunk = bytes >= 16 * mib ? kSlotBytes : std::min(mib, (bytes / 2 + 4095) & ~(size_t)4095);
     hipError_t err[kCopyThreads] = {};
     if (bytes >= 4 * mib) {
       std::thread helper[kCopyThreads];

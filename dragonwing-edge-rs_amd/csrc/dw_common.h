@@ -430,6 +430,9 @@ struct ResizeArgs {
 };
 void launch_resize_nearest(hipStream_t st, const ResizeArgs& a, int dtype);
 // Channel copy between views (concat/split when aliasing is impossible).
+// bytes from src to dst, either of which may be page-locked host memory; `done`
+// is recorded by the launch itself
+void launch_copy(hipStream_t st, const void* src, void* dst, unsigned bytes, hipEvent_t done);
 void launch_copy_channels(hipStream_t st, View src, View dst, int pixels, int channels, int esize);
 // Per-tensor min/max of an f32 view (calibration).  out: [min, max] floats,
 // must be initialised to (+inf, -inf) by the caller (done by launch_minmax_init).

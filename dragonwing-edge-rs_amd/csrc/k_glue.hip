@@ -6,6 +6,8 @@
 #include "dw_common.h"
 #include "dw_device.h"
 
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -627,6 +629,34 @@ void launch_copy_channels(hipStream_t st, View src, View dst, int pixels, int ch
   if (total == 0) return;
   hipLaunchKernelGGL(copy_channels_kernel, dim3(grid_for(total)), dim3(256), 0, st, src, dst, pixels,
                      channels * esize, esize);
+  DW_HIP(hipGetLastError());
+}
+
+namespace {
+// 16 bytes a thread where both ends are on 16-byte addresses (V = uint4, then
+// the tail), else one.
+template <typename V>
+__global__ __launch_bounds__(256) void copy_kernel(const V* __restrict__ src, V* __restrict__ dst, unsigned count,
+                                                   const uint8_t* __restrict__ tail_src, uint8_t* __restrict__ tail_dst,
+                                                   unsigned tail) {
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i < count) dst[i] = src[i];
+  if (i < tail) tail_dst[i] = tail_src[i];
+}
+}  // namespace
+
+void launch_copy(hipStream_t st, const void* src, void* dst, unsigned bytes, hipEvent_t done) {
+  const uint8_t* s = (const uint8_t*)src;
+  uint8_t* d = (uint8_t*)dst;
+  if (((uintptr_t)s | (uintptr_t)d) % 16 == 0) {
+    const unsigned count = bytes / 16;
+    hipExtLaunchKernelGGL(copy_kernel<uint4>, dim3(count / 256 + 1), dim3(256), 0, st, nullptr, done, 0,
+                          (const uint4*)s, (uint4*)d, count, s + 16 * (size_t)count, d + 16 * (size_t)count,
+                          bytes % 16);
+  } else {
+    hipExtLaunchKernelGGL(copy_kernel<uint8_t>, dim3(bytes / 256 + 1), dim3(256), 0, st, nullptr, done, 0, s, d, bytes,
+                          s, d, 0u);
+  }
   DW_HIP(hipGetLastError());
 }
 

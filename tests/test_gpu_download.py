@@ -13,7 +13,7 @@ MIB = 1 << 20
 DW_ERR_INVALID = -4
 
 
-@pytest.mark.parametrize("n", [1, 4095, 131073, MIB, MIB + 1, 4 * MIB - 1, 4 * MIB, 9 * MIB + 77,
+@pytest.mark.parametrize("n", [1, 4095, 16384, 16385, 131073, MIB, MIB + 1, 4 * MIB - 1, 4 * MIB, 9 * MIB + 77,
                                33 * MIB + 65537])
 def test_download_sizes(backend, n):
     src = np.random.default_rng(n).integers(0, 256, n).astype(np.uint8)
@@ -51,6 +51,25 @@ def test_sliced_tensors(backend, dtype, pixels):
         for name, w in zip(("r0", "r1", "y"), want):
             np.testing.assert_array_equal(rt.get_output_bytes(name).view(np_t).reshape(w.shape), w)
             np.testing.assert_array_equal(rt.get_output_f32(name, w.size).reshape(w.shape), w.astype(np.float32))
+
+
+def test_slice_off_16_byte_addresses(backend):
+    # one pixel of a slice is dense, from an address of its own: 6 bytes into the concat's output
+    xs = [np.random.default_rng(c).uniform(0.01, 2, (1, 1, 1, c)).astype(np.float16) for c in (3, 5000)]
+    g = Graph(GRAPH_F16)
+    for i, x in enumerate(xs):
+        g.add_tensor(f"x{i}", x.shape, "f16")
+        g.add_tensor(f"r{i}", x.shape, "f16")
+        g.add_op(f"relu{i}", "Relu", [f"x{i}"], [f"r{i}"])
+    g.add_tensor("y", (1, 1, 1, 5003), "f16")
+    g.add_op("cat", "Concat", ["r0", "r1"], ["y"], axis=3)
+    g.set_io(["x0", "x1"], ["y"])
+    rt = HipGraphRuntime(g, backend)
+    for i, x in enumerate(xs):
+        rt.set_input_bytes(f"x{i}", x)
+    rt.run()
+    for name, w in (("r0", xs[0]), ("r1", xs[1]), ("y", np.concatenate(xs, 3))):
+        np.testing.assert_array_equal(rt.get_output_bytes(name).view(np.float16), w.ravel())
 
 
 def test_null_destinations_are_refused(backend):

@@ -139,3 +139,14 @@ def test_conv_f32_past_the_tiles_offsets(backend):
         got = backend.to_numpy(by, np.float32, (h // 5, 5, 16384, 16))
         np.testing.assert_array_equal(got, np.broadcast_to(oracle.conv2d_f32_nhwc(block, w, (1, 1), (0, 0)), got.shape))
     assert times[1] < 6 * times[0]
+
+
+def test_download_of_64_kib(backend):
+    # through a kernel: little longer than 4 bytes, also where HIP's copies took 10 times as long, after a
+    # large allocation was freed
+    backend.from_numpy(np.ones(1 << 29, np.float32)).free()
+    times = []
+    for size in (4, 64 << 10):
+        buf, dst = backend.alloc(size), np.zeros(size, np.uint8)
+        times.append(per_call(backend, lambda: backend.download(buf, dst)))
+    assert times[1] < 2 * times[0]
