@@ -12,7 +12,6 @@
 
 #include <algorithm>
 #include <exception>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -53,6 +52,20 @@ void Backend::upload_async(void* dst, const void* src, size_t bytes) {
   DW_HIP(hipStreamSynchronize(stream));
 }
 
+// The first n slots; false if page-locked memory for them is refused.
+bool Backend::slots_ready(int n) {
+  for (int i = 0; i < n; ++i) {
+    Slot& s = slots[i];
+    if (!s.ev) DW_HIP(hipEventCreateWithFlags(&s.ev, hipEventDisableTiming));
+    if (!s.p && hipHostMalloc((void**)&s.p, kSlotBytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      s.p = nullptr;
+      return false;
+    }
+  }
+  return true;
+}
+
 // Chunks `thread`, thread + threads, ... of a download: the copy of one chunk
 // out of its page-locked slot runs while the device fills the thread's other
 // slot.  Every copy that was queued has ended when this returns.
@@ -62,9 +75,8 @@ hipError_t Backend::copy_chunks(uint8_t* dst, const uint8_t* src, size_t bytes, 
   const size_t n = (bytes + chunk - 1) / chunk;
   auto queue = [&](size_t c, int slot) -> hipError_t {
     const size_t len = std::min(chunk, bytes - c * chunk);
-    hipError_t e = hipMemcpyAsync(slots + (size_t)slot * kSlotBytes, src + c * chunk, len, hipMemcpyDeviceToHost,
-                                  stream);
-    return e == hipSuccess ? hipEventRecord(slot_ev[slot], stream) : e;
+    hipError_t e = hipMemcpyAsync(slots[slot].p, src + c * chunk, len, hipMemcpyDeviceToHost, stream);
+    return e == hipSuccess ? hipEventRecord(slots[slot].ev, stream) : e;
   };
   size_t next = (size_t)thread, done = next;  // the next chunk to queue, to copy out
   int in = 0, out = 0;                        // their places among the thread's two slots
@@ -75,9 +87,8 @@ hipError_t Backend::copy_chunks(uint8_t* dst, const uint8_t* src, size_t bytes, 
       next += (size_t)threads;
       in ^= 1;
     }
-    if (err == hipSuccess) err = hipEventSynchronize(slot_ev[first + out]);
-    if (err == hipSuccess)
-      memcpy(dst + done * chunk, slots + (size_t)(first + out) * kSlotBytes, std::min(chunk, bytes - done * chunk));
+    if (err == hipSuccess) err = hipEventSynchronize(slots[first + out].ev);
+    if (err == hipSuccess) memcpy(dst + done * chunk, slots[first + out].p, std::min(chunk, bytes - done * chunk));
     done += (size_t)threads;
     out ^= 1;
   }
@@ -93,60 +104,57 @@ hipError_t Backend::copy_chunks(uint8_t* dst, const uint8_t* src, size_t bytes, 
 // thing waited for: 64 KiB 12.8 us, 1 MiB 58 us.  HIP's copies of more than 16
 // KiB take 6 us longer there, or 110 us (seen after a 2 GB allocation was
 // freed), and those to ordinary memory 12.5 and 60 us, or 130 and 145.
+// Where no page-locked memory is to be had, HIP's copy to ordinary memory it is.
 void Backend::download(void* dst, const void* src, size_t bytes) {
+  const size_t mib = (size_t)1 << 20;
+  const int threads = bytes >= 4 * mib ? kCopyThreads : 1;
   hipPointerAttribute_t at{};
-  if (bytes && hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered) {
-    // memory the runtime knows (page-locked by the caller): the device copies there directly
-    DW_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
-  } else if (bytes) {
+  // memory the runtime knows (page-locked by the caller): the device copies there directly
+  bool direct = bytes && hipPointerGetAttributes(&at, dst) == hipSuccess && at.type != hipMemoryTypeUnregistered;
+  if (bytes && !direct) {
     (void)hipGetLastError();  // of an address that the runtime does not know
-    if (!slots) {
-      for (auto& e : slot_ev)
-        if (!e) DW_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-      DW_HIP(hipHostMalloc((void**)&slots, kSlots * kSlotBytes, hipHostMallocDefault));
-    }
-    uint8_t* d = (uint8_t*)dst;
-    const uint8_t* s = (const uint8_t*)src;
-    const size_t mib = (size_t)1 << 20;
-    if (bytes <= mib) {
-      launch_copy(stream, s, slots, (unsigned)bytes, slot_ev[0]);
-      DW_HIP(hipEventSynchronize(slot_ev[0]));
-      memcpy(d, slots, bytes);
-      return;
-    }
-    // a chunk costs about 10 us beside its bytes, which half a MiB hides; large
-    // downloads take whole slots
-    const size_t chunk = bytes >= 16 * mib ? kSlotBytes : std::min(mib, (bytes / 2 + 4095) & ~(size_t)4095);
-    hipError_t err[kCopyThreads] = {};
-    if (bytes >= 4 * mib) {
-      std::thread helper[kCopyThreads];
-      for (int t = 1; t < kCopyThreads; ++t) try {
-          helper[t] = std::thread([=, &err] { err[t] = copy_chunks(d, s, bytes, chunk, t, kCopyThreads); });
-        } catch (const std::system_error&) {
-          // no thread to be had: its share is copied below
-        }
-      err[0] = copy_chunks(d, s, bytes, chunk, 0, kCopyThreads);
-      for (int t = 1; t < kCopyThreads; ++t) {
-        if (helper[t].joinable())
-          helper[t].join();
-        else
-          err[t] = copy_chunks(d, s, bytes, chunk, t, kCopyThreads);
-      }
-    } else {
-      err[0] = copy_chunks(d, s, bytes, chunk, 0, 1);
-    }
-    for (hipError_t e : err) hip_check(e, "download");
+    direct = !slots_ready(bytes <= mib ? 1 : 2 * threads);
+  }
+  if (direct) DW_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
+  if (direct || !bytes) {
+    DW_HIP(hipStreamSynchronize(stream));
     return;
   }
-  DW_HIP(hipStreamSynchronize(stream));
+  uint8_t* d = (uint8_t*)dst;
+  const uint8_t* s = (const uint8_t*)src;
+  if (bytes <= mib) {
+    launch_copy(stream, s, slots[0].p, (unsigned)bytes, slots[0].ev);
+    DW_HIP(hipEventSynchronize(slots[0].ev));
+    memcpy(d, slots[0].p, bytes);
+    return;
+  }
+  // a chunk costs about 10 us beside its bytes, which half a MiB hides; large
+  // downloads take whole slots
+  const size_t chunk = bytes >= 16 * mib ? kSlotBytes : std::min(mib, (bytes / 2 + 4095) & ~(size_t)4095);
+  hipError_t err[kCopyThreads] = {};
+  std::thread helper[kCopyThreads];
+  for (int t = 1; t < threads; ++t) try {
+      helper[t] = std::thread([=, &err] { err[t] = copy_chunks(d, s, bytes, chunk, t, threads); });
+    } catch (const std::exception&) {
+      // no thread to be had: its share is copied below
+    }
+  err[0] = copy_chunks(d, s, bytes, chunk, 0, threads);
+  for (int t = 1; t < threads; ++t) {
+    if (helper[t].joinable())
+      helper[t].join();
+    else
+      err[t] = copy_chunks(d, s, bytes, chunk, t, threads);
+  }
+  for (hipError_t e : err) hip_check(e, "download");
 }
 
 Backend::~Backend() {
   if (stream) {
     (void)hipStreamSynchronize(stream);
-    if (slots) (void)hipHostFree(slots);
-    for (auto& e : slot_ev)
-      if (e) (void)hipEventDestroy(e);
+    for (auto& s : slots) {
+      if (s.p) (void)hipHostFree(s.p);
+      if (s.ev) (void)hipEventDestroy(s.ev);
+    }
     for (auto& w : ws)
       if (w.ptr) (void)hipFree(w.ptr);
     (void)hipStreamDestroy(stream);

@@ -69,11 +69,15 @@ struct Backend {
 
  private:
   // Page-locked slots that downloads go through, two for each copying thread
-  // (made by the first download, freed with the backend).
+  // (each made by the first download that wants it, freed with the backend).
   static constexpr int kCopyThreads = 4, kSlots = 2 * kCopyThreads;
   static constexpr size_t kSlotBytes = (size_t)2 << 20;
-  uint8_t* slots = nullptr;
-  hipEvent_t slot_ev[kSlots] = {};
+  struct Slot {
+    uint8_t* p = nullptr;
+    hipEvent_t ev = nullptr;
+  };
+  Slot slots[kSlots];
+  bool slots_ready(int n);
   hipError_t copy_chunks(uint8_t* dst, const uint8_t* src, size_t bytes, size_t chunk, int thread, int threads);
 };
 

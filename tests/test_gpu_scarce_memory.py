@@ -1,0 +1,67 @@
+"""Downloads where the runtime refuses more memory: each child process loads,
+ahead of the backend, a library whose hipHostMalloc and hipMalloc can be told to
+return hipErrorOutOfMemory."""
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = Path(__file__).resolve().parent.parent
+
+REFUSE = """
+#include <dlfcn.h>
+#include <stddef.h>
+int refuse_host, refuse_device, refused;
+static void* real(const char* name) {
+  static void* lib;
+  if (!lib) lib = dlopen("libamdhip64.so.7", RTLD_NOW);
+  return dlsym(lib, name);
+}
+static int no(void** p) { *p = 0; ++refused; return 2; }
+int hipHostMalloc(void** p, size_t n, unsigned flags) {
+  return refuse_host ? no(p) : ((int (*)(void**, size_t, unsigned))real("hipHostMalloc"))(p, n, flags);
+}
+int hipMalloc(void** p, size_t n) { return refuse_device ? no(p) : ((int (*)(void**, size_t))real("hipMalloc"))(p, n); }
+"""
+
+SETUP = """
+import ctypes as C
+import sys
+sys.path.insert(0, {root!r})
+lib = C.CDLL({lib!r}, C.RTLD_GLOBAL)
+flag = lambda name: C.c_int.in_dll(lib, name)
+import numpy as np
+import __graft_entry__
+__graft_entry__.import_pkg()
+import dragonwing_edge_rs_amd as dw
+from dragonwing_edge_rs_amd.graph import GRAPH_F32, Graph, HipGraphRuntime
+be = dw.Backend(0)
+"""
+
+HOST = """
+sizes = (5, 300001, (2 << 20) + 3, (9 << 20) + 77)
+srcs = [np.random.default_rng(n).integers(0, 256, n).astype(np.uint8) for n in sizes]
+bufs = [be.from_numpy(s) for s in srcs]
+for refuse in (1, 0, 1):
+    flag("refuse_host").value = refuse
+    for b, s in zip(bufs, srcs):
+        np.testing.assert_array_equal(be.to_numpy(b, np.uint8, s.shape), s)
+assert flag("refused").value >= len(sizes)
+"""
+
+
+def run(tmp_path, body):
+    lib = tmp_path / "refuse.so"
+    (tmp_path / "refuse.c").write_text(REFUSE)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(tmp_path / "refuse.c"), "-ldl"], check=True)
+    code = SETUP.format(root=str(ROOT), lib=str(lib)) + body
+    r = subprocess.run([sys.executable, "-c", code], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
+                       timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
+def test_download_without_page_locked_memory(tmp_path):
+    run(tmp_path, HOST)
