@@ -216,7 +216,7 @@ __device__ __forceinline__ void epilogue4(const IgemmArgs& a, const EpiLds& e, c
     if (a.act == ACT_SILU) {
       p01 = silu_f16_pk_lite(p01);
       p23 = silu_f16_pk_lite(p23);
-    } else if (a.act != ACT_NONE) {
+    } else if (a.act == ACT_RELU) {
       p01 = pk_make(f16_act_bits(pk_lo(p01), ACT_RELU), f16_act_bits(pk_hi(p01), ACT_RELU));
       p23 = pk_make(f16_act_bits(pk_lo(p23), ACT_RELU), f16_act_bits(pk_hi(p23), ACT_RELU));
     }
@@ -453,7 +453,7 @@ __device__ __forceinline__ bool igemm_store_f16(const IgemmArgs& a, const EpiLds
         v[cb][0] = silu_f16_pk_lite(v[cb][0]);
         v[cb][1] = silu_f16_pk_lite(v[cb][1]);
       }
-    } else if (a.act != ACT_NONE) {
+    } else if (a.act == ACT_RELU) {
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb)
 #pragma unroll

@@ -334,12 +334,12 @@ __global__ __launch_bounds__(256) void dwconv3_kernel(const Dw3Args p) {
 
 template <bool H, int SW, bool ROW1>
 void launch_act(hipStream_t st, const Dw3Args& p, unsigned blocks) {
-  if (p.d.act == ACT_NONE)
-    hipLaunchKernelGGL((dwconv3_kernel<H, SW, ROW1, ACT_NONE>), dim3(blocks), dim3(256), 0, st, p);
-  else if (p.d.act == ACT_RELU)
+  if (p.d.act == ACT_RELU)
     hipLaunchKernelGGL((dwconv3_kernel<H, SW, ROW1, ACT_RELU>), dim3(blocks), dim3(256), 0, st, p);
   else if (p.d.act == ACT_SILU)
     hipLaunchKernelGGL((dwconv3_kernel<H, SW, ROW1, ACT_SILU>), dim3(blocks), dim3(256), 0, st, p);
+  else if (!H || p.d.act == ACT_NONE)  // (f32: a value that names no activation is none, as in dwconv_kernel)
+    hipLaunchKernelGGL((dwconv3_kernel<H, SW, ROW1, ACT_NONE>), dim3(blocks), dim3(256), 0, st, p);
   else
     fail(-2, "depthwise: no kernel for this activation");
 }
