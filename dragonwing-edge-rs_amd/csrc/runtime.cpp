@@ -3167,7 +3167,17 @@ static void download_tensor(dw::Runtime& rt, const dw::RtTensor& t, void* dst) {
   hipStream_t st = rt.be->stream;
   const uint8_t* src = (const uint8_t*)t.base + (size_t)t.abs_off * es;
   if (t.pix_stride != t.c && t.pixels() > 1) {
-    void* dense = rt.be->workspace(dw::Backend::WS_POST, t.bytes());
+    void* dense = nullptr;
+    try {
+      dense = rt.be->workspace(dw::Backend::WS_POST, t.bytes());
+    } catch (const dw::Error&) {
+      // no device memory to gather into: the strided copy
+      (void)hipGetLastError();
+      DW_HIP(hipStreamSynchronize(st));
+      DW_HIP(hipMemcpy2D(dst, t.c * es, src, (size_t)t.pix_stride * es, t.c * es, (size_t)t.pixels(),
+                         hipMemcpyDeviceToHost));
+      return;
+    }
     dw::launch_copy_channels(st, t.view(), {dense, (int)t.c, 0}, (int)t.pixels(), (int)t.c, (int)es);
     src = (const uint8_t*)dense;
   }

@@ -52,6 +52,30 @@ for refuse in (1, 0, 1):
 assert flag("refused").value >= len(sizes)
 """
 
+# a slice of the concat's channels, read back once without memory to gather into and once with it
+DEVICE = """
+xs = [np.random.default_rng(c).uniform(0.1, 1, (2, 9, 7, c)).astype(np.float32) for c in (12, 20)]
+g = Graph(GRAPH_F32)
+for i, x in enumerate(xs):
+    g.add_tensor(f"x{i}", x.shape)
+    g.add_tensor(f"r{i}", x.shape)
+    g.add_op(f"relu{i}", "Relu", [f"x{i}"], [f"r{i}"])
+g.add_tensor("y", (2, 9, 7, 32))
+g.add_op("cat", "Concat", ["r0", "r1"], ["y"], axis=3)
+g.set_io(["x0", "x1"], ["y"])
+rt = HipGraphRuntime(g, be)
+for i, x in enumerate(xs):
+    rt.set_input_f32(f"x{i}", x)
+rt.run()
+before = flag("refused").value
+for refuse in (1, 0):
+    flag("refuse_device").value = refuse
+    for i, x in enumerate(xs):
+        np.testing.assert_array_equal(rt.get_output_f32(f"r{i}", x.size).reshape(x.shape), x)
+    rt.run()
+assert flag("refused").value > before
+"""
+
 
 def run(tmp_path, body):
     lib = tmp_path / "refuse.so"
@@ -65,3 +89,7 @@ def run(tmp_path, body):
 
 def test_download_without_page_locked_memory(tmp_path):
     run(tmp_path, HOST)
+
+
+def test_sliced_output_without_device_memory(tmp_path):
+    run(tmp_path, DEVICE)
