@@ -141,6 +141,30 @@ def test_conv_f32_past_the_tiles_offsets(backend):
     assert times[1] < 6 * times[0]
 
 
+# in workgroups of one wave with 16 loads a value, whatever there is to load: 2.2 to 2.5 times as long as the relu
+@pytest.mark.parametrize("dtype", [ops.DTYPE_F32, ops.DTYPE_F16])
+@pytest.mark.parametrize("n,h,w,c", [(4096, 1, 1, 1024), (4096, 2, 1, 1021), (2500, 3, 1, 1030)])
+def test_pool_of_few_pixels(backend, n, h, w, c, dtype):
+    f16 = dtype == ops.DTYPE_F16
+    x = np.random.default_rng(c).normal(0, 2, (n, h, w, c)).astype(np.float16 if f16 else np.float32)
+    bx, by = backend.from_numpy(x), backend.alloc(n * c * x.itemsize)
+    t = per_call(backend, lambda: ops.global_avg_pool_nhwc(backend, dtype, bx, by, n, h, w, c))
+    assert t < 1.6 * relu_time(backend, n * c * (h * w + 1) // 2)
+    if f16:
+        x = x.view(np.uint16)
+    want = (oracle.global_avg_pool_fp16 if f16 else oracle.global_avg_pool_f32)(x)
+    np.testing.assert_array_equal(backend.to_numpy(by, x.dtype, (n, c)), want)
+
+
+# byte a thread (up to 4 pixels, or channels in no fours) in both workgroup sizes, and a dword
+@pytest.mark.parametrize("n,h,w,c", [(4096, 2, 2, 67), (70, 1, 3, 260), (4099, 5, 1, 65), (5, 5, 1, 64)])
+def test_quantized_pool_of_few_pixels(backend, n, h, w, c):
+    x = np.random.default_rng(c).integers(0, 256, (n, h, w, c)).astype(np.uint8)
+    by = backend.alloc(n * c)
+    ops.qlinear_global_avg_pool_u8(backend, backend.from_numpy(x), by, n, h, w, c, 0.03, 125, 0.01, 128)
+    np.testing.assert_array_equal(backend.to_numpy(by, np.uint8, (n, c)), oracle.qlinear_gap_u8(x, 0.03, 125, 0.01, 128))
+
+
 def test_download_of_64_kib(backend):
     # through a kernel: little longer than 4 bytes, also where HIP's copies took 10 times as long, after a
     # large allocation was freed
