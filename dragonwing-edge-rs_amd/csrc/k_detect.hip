@@ -29,6 +29,8 @@
 #include "dw_common.h"
 #include "dw_device.h"
 
+#include <type_traits>
+
 namespace dw {
 namespace {
 
@@ -120,12 +122,14 @@ __global__ __launch_bounds__(256) void detect_tail_tile_kernel(TailLevels L, flo
   const int dw = H ? chans / 2 : chans, pixdw = H ? L.pix[s] / 2 : L.pix[s];
   const uint32_t* x = (const uint32_t*)L.x[s] + ((size_t)b * hw + a0) * (size_t)pixdw;
   const int sa = 256 / dw, sr = 256 % dw;
-  {
-    constexpr int kTailLoads = tail_loads(H);
-    uint32_t v[kTailLoads];
+  // all of a thread's dwords on their way before the first is stored: N of them,
+  // for the tiles that have few (few channels, or a map's last tile)
+  auto stage = [&](auto count) {
+    constexpr int N = decltype(count)::value;
+    uint32_t v[N];
     int a = t / dw, r = t % dw;
 #pragma unroll
-    for (int i = 0; i < kTailLoads; ++i) {
+    for (int i = 0; i < N; ++i) {
       v[i] = x[a < live ? (size_t)a * pixdw + r : 0];
       a += sa;
       r += sr;
@@ -137,7 +141,7 @@ __global__ __launch_bounds__(256) void detect_tail_tile_kernel(TailLevels L, flo
     a = t / dw;
     r = t % dw;
 #pragma unroll
-    for (int i = 0; i < kTailLoads; ++i) {
+    for (int i = 0; i < N; ++i) {
       if (a < live) {
         if constexpr (H) {
           tile[a * ld + 2 * r] = h2f((uint16_t)v[i]);
@@ -153,7 +157,13 @@ __global__ __launch_bounds__(256) void detect_tail_tile_kernel(TailLevels L, flo
         ++a;
       }
     }
-  }
+  };
+  if (live * dw <= 2 * 256)
+    stage(std::integral_constant<int, 2>{});
+  else if (live * dw <= 8 * 256)
+    stage(std::integral_constant<int, 8>{});
+  else
+    stage(std::integral_constant<int, tail_loads(H)>{});
   __syncthreads();
   const float* row = tile + min(lane, live - 1) * ld;  // idle lanes repeat the last anchor
   dist[wave * 64 + lane] = dfl_side<R>(reg_max, [&](int k) { return row[wave * reg_max + k]; });
@@ -170,8 +180,9 @@ __global__ __launch_bounds__(256) void detect_tail_tile_kernel(TailLevels L, flo
   if (lane < live) o[(size_t)wave * A] = v;
 }
 
-// Any head (channels that do not pair into dwords, or more than a thread of
-// the tile kernel holds): a thread per anchor, straight from memory.
+// A thread per anchor, straight from memory: any head (channels that do not
+// pair into dwords, or more than a thread of the tile kernel holds), and those
+// that tail_by_tiles leaves to it.
 template <bool H>
 __global__ __launch_bounds__(256) void detect_tail_kernel(TailLevels L, float* out, int nc, int reg_max) {
   const int a = blockIdx.x * 256 + threadIdx.x;
@@ -501,6 +512,28 @@ __global__ __launch_bounds__(kNmsThreads) void pp_nms_kernel(PPArgs p) {
     }
 }
 
+// Whether the tiles are expected to be done before a thread per anchor, in
+// microseconds: their workgroups, each of which has a start and costs by its
+// channels however few its anchors are, against the waves that walk every
+// channel of their anchors (and a side's logits three times).  Fitted (14-30%) to
+// 12 heads of 6 to 144 channels on 12 batches of 1 to 20000 images with 1 to
+// 8400 anchors, both kernels timed at each; the thread has the benefit of the
+// doubt, which leaves the choice at most 1.2x from it.  20000 images of 3
+// anchors, 6 channels in f32: 18.5 against 67 us (1 x 8400 of 144: 47 against
+// 12); 32 of 8400 anchors, 6 channels 7.4 against 10.5 us.
+bool tail_by_tiles(int dtype, int n, int anchors, int tiles, int reg_max, int chans) {
+  const float k = (float)n / 1000.0f, wg = k * (float)tiles, all = k * (float)anchors, ch = (float)chans;
+  const float blocks = k * (float)((anchors + 255) / 256), waves = k * (float)((anchors + 63) / 64);
+  const bool h = dtype == F16;
+  const float tile = h ? 6.6f + wg * (0.75f + 0.0354f * ch) + 0.00029f * all * ch + 0.0051f * ch
+                       : 6.5f + wg * (0.82f + 0.0390f * ch) + 0.00093f * all * ch + 0.0073f * ch;
+  const float thread = h ? 3.5f + 0.22f * blocks + 0.0578f * waves * ch + 0.0007f * all * ch + 0.1925f * ch +
+                               0.118f * waves * (float)reg_max
+                         : 4.0f + 0.0566f * waves * ch + 0.0027f * all * ch + 0.1621f * ch +
+                               0.083f * waves * (float)reg_max;
+  return 1.2f * tile <= thread;
+}
+
 }  // namespace
 
 void launch_detect_tail(hipStream_t st, int dtype, const DetectTailArgs& t, float* out, int n) {
@@ -530,7 +563,7 @@ void launch_detect_tail(hipStream_t st, int dtype, const DetectTailArgs& t, floa
     tiles += (t.h[s] * t.w[s] + kTailAnchors - 1) / kTailAnchors;
     tile = tile && (t.pix[s] * es) % 4 == 0 && (uintptr_t)t.x[s] % 4 == 0;
   }
-  if (tile) {
+  if (tile && tail_by_tiles(dtype, n, a, tiles, t.reg_max, chans)) {
     auto* k = dtype == F16 ? (t.reg_max == 16 ? detect_tail_tile_kernel<true, 16> : detect_tail_tile_kernel<true, 0>)
                            : (t.reg_max == 16 ? detect_tail_tile_kernel<false, 16> : detect_tail_tile_kernel<false, 0>);
     hipLaunchKernelGGL(k, dim3((unsigned)tiles, (unsigned)n), dim3(256), lds, st, L, out, t.nc, t.reg_max);

@@ -165,6 +165,25 @@ def test_quantized_pool_of_few_pixels(backend, n, h, w, c):
     np.testing.assert_array_equal(backend.to_numpy(by, np.uint8, (n, c)), oracle.qlinear_gap_u8(x, 0.03, 125, 0.01, 128))
 
 
+# in tiles of 64 anchors with the loads of 160 channels: 46 and 4.5 times as long as the relu
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("n,hw,nc,reg_max,limit", [(20000, [(1, 2), (1, 1)], 2, 2, 12),
+                                                   (32, [(80, 80), (40, 40), (20, 20)], 2, 1, 3)])
+def test_tail_of_few_channels(backend, n, hw, nc, reg_max, limit, f16):
+    from test_gpu_detect_edges import f64_tail
+    r = np.random.default_rng(n)
+    strides = [8.0 * 2 ** i for i in range(len(hw))]
+    A, chans = sum(h * w for h, w in hw), 4 * reg_max + nc
+    lv = [r.normal(0, 3, (n, h, w, chans)).astype(np.float16 if f16 else np.float32) for h, w in hw]
+    bl, out = [backend.from_numpy(x) for x in lv], backend.alloc(n * (4 + nc) * A * 4)
+    t = per_call(backend, lambda: ops.yolo_detect_tail(backend, bl, hw, strides, n, out, nc=nc, reg_max=reg_max,
+                                                       dtype=ops.DTYPE_F16 if f16 else ops.DTYPE_F32))
+    assert t < limit * relu_time(backend, n * A * chans)
+    got = backend.to_numpy(out, np.float32, (n, 4 + nc, A)).astype(np.float64)
+    ref = f64_tail([x.astype(np.float64) for x in lv], strides, nc, reg_max)
+    assert (np.abs(got - ref) <= 1e-5 * np.abs(ref).max(axis=(0, 2), keepdims=True)).all()  # as test_tail_tiles
+
+
 def test_download_of_64_kib(backend):
     # through a kernel: little longer than 4 bytes, also where HIP's copies took 10 times as long, after a
     # large allocation was freed
