@@ -410,6 +410,9 @@ float fp_cost(const IgemmArgs& a, int bc, int waves) {
 // weight slice of the channel tile is staged in chunks of at most kWeightLds
 // bytes.
 TileCfg pick_any(const IgemmArgs& a);
+struct TilePick {
+  int bc, pb, tpw;
+};
 
 // A launch that also writes an upsampled copy (a.y_up) takes any tile whose
 // epilogue is igemm_store's; the persistent small-K kernel's is its own, so
@@ -469,11 +472,12 @@ TileCfg pick_any(const IgemmArgs& a) {
   // The widest channel tile and the widest pixel tile (16 * pb pixels per
   // wave) that still gives about two workgroups per CU reads the input least
   // often, but leaves CUs idle on small maps and makes long workgroups of
-  // deep layers; it stays unless another tile is expected to take under 95%
-  // of its time.  On 250 convolutions kept out of the fits the choice is 1.16x
-  // faster (geometric mean) and 4.3% off the best tile; 1-2% of them are more
-  // than 3% slower, the worst 9%.  20 x 20, 256 -> 256 3x3, one image: 15.8
-  // -> 9.2 us.
+  // deep layers; it stays unless another tile is expected to take clearly less
+  // (how clearly stands below).  On 5000 convolutions kept out of the fits
+  // (those above and 5x5, up to 720 channels) the choice is 1.22x faster
+  // (geometric mean), 0.5% of them are more than 3% slower, the worst 14%; with
+  // 95% of its time enough for every tile that was 2.3%, the worst 36%.  20 x
+  // 20, 256 -> 256 3x3, one image: 15.8 -> 9.2 us.
   const int bc = channel_tile(a.cout);
   const int ctiles = a.cout_pad / bc;
   TileCfg best = make_tile(a, bc, 1);
@@ -488,14 +492,13 @@ TileCfg pick_any(const IgemmArgs& a) {
   const int esize = a.epi == EPI_F16 ? 2 : 1;
   // 64 PB-pixel tiles: (m + 64 PB - 1) / (64 PB) for PB = 1, 2, 4
   auto pixel_tiles = [&](int pb) { return (a.m + 64 * pb - 1) >> (pb == 4 ? 8 : pb == 2 ? 7 : 6); };
-  float least = 0.95f * tile_cost(esize, 0, a.ksteps, best.bc, best.pb, pixel_tiles(best.pb) * ctiles);
-  int b_bc = 0, b_pb = 0, b_tpw = 0;  // the best so far, if not `best`
+  const float base = tile_cost(esize, 0, a.ksteps, best.bc, best.pb, pixel_tiles(best.pb) * ctiles);
+  float least = 0.95f * base;
+  TilePick f{};
   auto consider = [&](float c, int b, int p, int tpw) {
     if (c < least) {
       least = c;
-      b_bc = b;
-      b_pb = p;
-      b_tpw = tpw;
+      f = {b, p, tpw};
     }
   };
   for (int b : {128, 96, 80, 64, 48, 32, 16}) {
@@ -510,6 +513,18 @@ TileCfg pick_any(const IgemmArgs& a) {
   }
   for (int b : {256, 128, 64})
     if (wide_ok(a, b)) consider(tile_cost(esize, 2, a.ksteps, b, 4, pixel_tiles(4) * (a.cout_pad / b)), b, 4, -3);
+  // A tile of 64 pixels in place of one, or the wide kernel's, is believed at 95%
+  // (at 85 to 95% 1% of 690 such choices were more than 3% slower); one of more
+  // pixels, or of fewer than the first's, is not (22% of 430), the streamed
+  // kernel's least; and K beyond the fits, which end at 512 channels of 3x3,
+  // counts for less.
+  const bool deep = a.ksteps > (esize == 1 ? 72 : 144);
+  const bool near = f.tpw == -3 || (f.pb == 1 && best.pb == 1);
+  const float enough = deep ? 0.7f : near ? 0.95f : f.tpw == -1 ? 0.8f : 0.85f;
+  if (f.bc && least >= enough * base) {
+    least = 0.95f * base;
+    f = {};
+  }
   // Tiles of 16 pixels where they are few, against 95% of the best above
   // (least when nothing above was chosen is that already).
   // Split K (int8: a sum of integers is the same in any order; fp16 layers
@@ -519,7 +534,8 @@ TileCfg pick_any(const IgemmArgs& a) {
   // In order (fp16): half of 29 layers of up to 1024 such waves, those 1.37x
   // faster; below four k-steps there is no chain to shorten (7 x 21 96 -> 92
   // 1x1 of 5 images: 4.8 against 3.9 us).
-  if (b_bc) least *= 0.95f;
+  if (f.bc) least *= 0.95f;
+  if (deep) least = std::min(least, 0.7f * base);
   const int p16 = (a.m + 15) >> 4;
   for (int b : {16, 32, 64}) {
     if (a.cout_pad % b != 0) continue;
@@ -529,15 +545,16 @@ TileCfg pick_any(const IgemmArgs& a) {
       if (a.ksteps >= 4 && fp_ok(a, b)) consider(fp_cost(a, b, (int)tiles), b, 1, -7);
     } else {
       for (int nw : {4, 8, 16})
-        if (ks_ok(a, b, nw)) consider(ks_cost(a, b, nw, (int)tiles), b, nw, -6);
+        if (ks_ok(a, b, nw))  // (four workgroups a CU are short of loads: up to 18% slower than expected to win by 25%)
+          consider(ks_cost(a, b, nw, (int)tiles) * (tiles > 768 ? 1.3f : 1.0f), b, nw, -6);
     }
   }
-  if (!b_bc) return best;
-  return b_tpw == 0    ? make_tile(a, b_bc, b_pb)
-         : b_tpw == -1 ? make_st_tile(a, b_bc, b_pb)
-         : b_tpw == -3 ? make_wide_tile(a, b_bc)
-         : b_tpw == -6 ? make_ks_tile(a, b_bc, b_pb)
-                       : make_fp_tile(a, b_bc);
+  if (!f.bc) return best;
+  return f.tpw == 0    ? make_tile(a, f.bc, f.pb)
+         : f.tpw == -1 ? make_st_tile(a, f.bc, f.pb)
+         : f.tpw == -3 ? make_wide_tile(a, f.bc)
+         : f.tpw == -6 ? make_ks_tile(a, f.bc, f.pb)
+                       : make_fp_tile(a, f.bc);
 }
 
 // Epilogue specialisation for the arguments.

@@ -184,6 +184,35 @@ def test_tail_of_few_channels(backend, n, hw, nc, reg_max, limit, f16):
     assert (np.abs(got - ref) <= 1e-5 * np.abs(ref).max(axis=(0, 2), keepdims=True)).all()  # as test_tail_tiles
 
 
+# the widest tile of at least 512 workgroups, which wider ones were chosen over: 1.19 to 1.36 times as long
+@pytest.mark.parametrize("f16,x_shape,w_shape,s,tile", [
+    (True, (27, 158, 30, 352), (5, 5, 352, 32), 1, "32,2"), (True, (1, 156, 128, 216), (1, 1, 216, 532), 2, "128,1"),
+    (True, (14, 30, 77, 16), (3, 3, 16, 204), 1, "128,1"), (False, (16, 13, 151, 384), (1, 1, 384, 428), 2, "128,1"),
+    (False, (25, 14, 85, 608), (5, 5, 608, 36), 1, "48,1")])
+def test_chosen_tile_is_not_slower(backend, monkeypatch, f16, x_shape, w_shape, s, tile):
+    (n, h, w, ci), (k, _, _, co) = x_shape, w_shape
+    ho, wo = oracle.out_hw(h, w, k, k, s, s, k // 2, k // 2)
+    bx, bw = (backend.from_numpy(np.ones(sh, np.float16 if f16 else np.int8)) for sh in (x_shape, w_shape))
+    by = backend.alloc(n * ho * wo * co * (2 if f16 else 4))
+    geo = (by, n, h, w, ci, co, k, k, s, s, k // 2, k // 2)
+
+    def conv():
+        if f16:
+            ops.conv2d_bias_act_f16_nhwc(backend, bx, bw, None, *geo)
+        else:
+            ops.conv2d_i8_nhwc(backend, bx, bw, *geo)
+
+    times = [np.inf, np.inf]
+    for _ in range(2):
+        for i in (0, 1):
+            if i:
+                monkeypatch.setenv("DW_IGEMM_TILE", tile)
+            else:
+                monkeypatch.delenv("DW_IGEMM_TILE", raising=False)
+            times[i] = min(times[i], per_call(backend, conv, calls=20))
+    assert times[0] < 1.12 * times[1]
+
+
 def test_download_of_64_kib(backend):
     # through a kernel: little longer than 4 bytes, also where HIP's copies took 10 times as long, after a
     # large allocation was freed
