@@ -175,21 +175,33 @@ __global__ __launch_bounds__(256) void gemm_thread_kernel(const void* A, const v
 }
 
 // Whether a thread per output is expected to be done before the tiles, in
-// microseconds: its workgroups' dispatch, or a chain of K steps that the waves
-// in flight lengthen, against the tiles' workgroups.  Fitted to 9 shapes of up
-// to 6.5M outputs with K of 1 to 128, both kernels timed at each: 1024 x 1024
-// f32 with K = 8 4.4 against 17.9 us, with K = 64 14.9 against 20.6 us; 65535 x
-// 100 with K = 32 67 against 114 us; 32 x 1000 with K = 8 3.9 against 3.6 us,
-// with K = 128 13.8 against 3.8 us.  Above 64 steps it won nowhere by more
-// than 6%.
+// microseconds: a chain of K steps that the waves in flight lengthen (of a
+// transposed B, the more so the further apart its rows lie), against the tiles'
+// workgroups, and their chains where they fill the chip more than once.  Fitted
+// (7-30%) to 746 products of up to 4096 rows and 8192 columns with K of 8 to
+// 290, both kernels timed at each; the thread has the benefit of the doubt.  The
+// choice is more than 5% slower than a thread per output in 6 of them, the
+// worst 19%.  1024 x 1024 f32 with K = 8
+// 4.4 against 17.9 us, with K = 64 14.9 against 20.6 us; 3721 x 1616 with K = 75
+// 104 against 120 us; 32 x 1000 with K = 8 3.9 against 3.6 us, with K = 128 13.8
+// against 3.8 us.  Above 128 steps it won nowhere.
 bool gemm_by_threads(int dtype, bool trans_b, int m, int n, int k) {
-  if (k > 64) return false;
-  const float waves = (float)m * (float)((n - 1) / 64 + 1), blocks = (float)m * (float)((n - 1) / 256 + 1);
-  const float tiles = (float)((m - 1) / kGemmR + 1) * (float)((n - 1) / kGemmC + 1);
-  const float chain = 2.6f + (float)k * std::max(0.09f, (trans_b ? 1e-4f : 1.3e-5f) * waves);
-  const float t = std::max(std::max(3.8f, 0.00047f * blocks), chain);
-  const float per_tile = dtype == F32 ? (trans_b ? 0.0026f : 0.00172f) : (trans_b ? 0.003f : 0.00245f);
-  return t < std::max(3.6f, 2.3f + per_tile * tiles + 7e-6f * tiles * (float)k);
+  if (k > 128) return false;
+  struct Fit {
+    float start, tile, step, round;  // tiles: a call, a tile, its step, a step of 1024 tiles
+    float tstart, tstep, wave;       // threads: a call, a step, a wave's step
+  };
+  static const Fit fits[2][2] = {{{3.59f, 1.65e-3f, 6.93e-6f, 1.77e-3f, 2.29f, 0.0654f, 1.12e-5f},
+                                  {2.94f, 2.33e-3f, 8.9e-6f, 1.07e-2f, 1.76f, 0.0756f, 5.7e-5f}},
+                                 {{3.44f, 2.43e-3f, 2.72e-6f, 3.88e-3f, 2.13f, 0.0839f, 1.5e-5f},
+                                  {3.0f, 2.43e-3f, 9.8e-6f, 1.36e-2f, 1.83f, 0.082f, 5.7e-5f}}};
+  const Fit& f = fits[dtype == F16][trans_b];
+  const int rows = (m - 1) / kGemmR + 1, cols = (n - 1) / kGemmC + 1;
+  const float tiles = (float)rows * (float)cols, rounds = (float)(((long long)rows * cols + 1023) / 1024);
+  const float steps = (float)k, row_bytes = steps * (dtype == F16 ? 2.0f : 4.0f);
+  const float waves = (float)m * (float)((n - 1) / 64 + 1) * (trans_b ? std::max(1.0f, row_bytes / 36.0f) : 1.0f);
+  return f.tstart + steps * (f.tstep + f.wave * waves) <
+         (trans_b ? 1.1f : 1.05f) * (f.start + tiles * (f.tile + f.step * steps) + f.round * steps * rounds);
 }
 
 // int32 sum of i8 products (gemm_i8_scalar, ops.rs:2981-2995); integer

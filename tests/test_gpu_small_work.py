@@ -61,10 +61,11 @@ def test_gemm_of_few_steps(backend, m, n, k, f16):
     np.testing.assert_array_equal(backend.to_numpy(bc, a.dtype, (m, n)), want(a, b))
 
 
+# (10 steps: in tiles 7 times as long)
 @pytest.mark.parametrize("f16", [False, True])
-def test_transposed_gemm_of_few_steps(backend, f16):
+@pytest.mark.parametrize("m,n,k,limit", [(1500, 700, 4, 3), (523, 2525, 10, 5)])
+def test_transposed_gemm_of_few_steps(backend, m, n, k, limit, f16):
     from oracle.cpu_graph import CpuGraph
-    m, n, k = 1500, 700, 4
     r = np.random.default_rng(k + f16)
     dt, cast = ("f16", lambda v: v.astype(np.float16).view(np.uint16)) if f16 else ("f32", lambda v: v.astype(np.float32))
     x, w, b = cast(r.normal(0, 1, (m, k))), cast(r.normal(0, 0.2, (n, k))), cast(r.normal(0, 1, n))
@@ -77,7 +78,7 @@ def test_transposed_gemm_of_few_steps(backend, f16):
     g.set_io(["x"], ["y"])
     rt = HipGraphRuntime(g, backend)
     rt.set_input_bytes("x", x)
-    assert per_call(backend, rt.run) < 3 * relu_time(backend, m * n)
+    assert per_call(backend, rt.run) < limit * relu_time(backend, m * n)
     cg = CpuGraph(g.to_dict(), g.initializer)
     cg.set_input("x", x)
     np.testing.assert_array_equal(rt.get_output_bytes("y").view(x.dtype).reshape(m, n), cg.run()["y"])
