@@ -236,18 +236,25 @@ __global__ __launch_bounds__(T) void global_avg_pool_kernel(const void* X, void*
   const int b = blockIdx.y;
   if (ch >= c || b >= n) return;
   const E* x = (const E*)X + (size_t)b * hw * c + ch;
+  auto widen = [](E v) -> float {
+    if constexpr (F16) return h2f(v);
+    return v;
+  };
   float sum = 0.0f;
-  for (unsigned s0 = 0; s0 < (unsigned)hw; s0 += AHEAD) {
+  unsigned s0 = 0;
+  for (; s0 + AHEAD <= (unsigned)hw; s0 += AHEAD) {
+    E v[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) v[j] = x[(size_t)(s0 + j) * c];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) sum += widen(v[j]);
+  }
+  if (AHEAD > 1 && s0 < (unsigned)hw) {
     E v[AHEAD];
 #pragma unroll
     for (int j = 0; j < AHEAD; ++j) v[j] = x[(size_t)umin(s0 + j, hw - 1) * c];
 #pragma unroll
-    for (int j = 0; j < AHEAD; ++j) {
-      float f;
-      if constexpr (F16) f = h2f(v[j]);
-      else f = v[j];
-      sum = s0 + j < (unsigned)hw ? sum + f : sum;
-    }
+    for (int j = 0; j < AHEAD; ++j) sum = s0 + j < (unsigned)hw ? sum + widen(v[j]) : sum;
   }
   const float mean = __fdiv_rn(sum, (float)hw);
   if constexpr (F16)
