@@ -252,7 +252,11 @@ bool launch_conv1x1_exact(hipStream_t st, const DirectArgs& a);
 int conv1x1_exact_channels(const DirectArgs& a);
 // The register-tiled kernel, f32 in and out, any shape (k_conv_f32.hip).
 bool conv_f32_reaches(const DirectArgs& a);  // its 32-bit offsets do
-float conv_f32_cost(const DirectArgs& a);    // expected microseconds, of layers of few channels
+struct CfWindow {
+  int kh0, kh, kw0, kw;  // the rows and columns of the filter that meet the image at some output
+};
+CfWindow conv_f32_window(const DirectArgs& a);
+float conv_f32_cost(const DirectArgs& a, const CfWindow& w);  // expected microseconds, of layers of few channels
 void launch_conv_f32(hipStream_t st, const DirectArgs& a);
 
 }  // namespace dw

@@ -43,6 +43,7 @@ struct CfArgs {
   int taps_chunk;  // segments in a chunk
   int segs_tap;    // segments of a tap (1 if whole taps fit)
   int chunks;
+  int wtap, wrow;  // weights between two taps, and more between two rows of them
   int act;
   int x_bytes, w_bytes;
 };
@@ -104,7 +105,7 @@ __global__ __launch_bounds__(256, (CfTile<PX, CH, VEC>::kWaves)) void conv_f32_k
 #pragma unroll
   for (int i = 0; i < T::kWLoads; ++i) {
     const int idx = t + 256 * i, k = idx / T::kCh, tl = k / a.segp;
-    wo[i] = (tl * a.cin + k - tl * a.segp) * a.cout + c0 + idx % T::kCh;
+    wo[i] = tl * a.wtap + (k - tl * a.segp) * a.cout + c0 + idx % T::kCh;
   }
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, a.x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)a.w, (short)0, a.w_bytes, 0x00020000);
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(256, (CfTile<PX, CH, VEC>::kWaves)) void conv_f32_k
     const int tap = tap0 + ktl;
     const int kh = tap / a.kw, kw = tap - kh * a.kw;
     const int koff = (kh * a.wd + kw) * a.xs + ic0 + kic;
-    const int woff = (tap0 * a.cin + ic0) * a.cout;
+    const int woff = tap0 * a.wtap + tap0 / a.kw * a.wrow + ic0 * a.cout;
 #pragma unroll
     for (int i = 0; i < T::kXLoads; ++i) {
       if constexpr (VEC)
@@ -245,8 +246,10 @@ void launch_tile(hipStream_t st, CfArgs a) {
   a.seg = whole ? a.cin : T::kK;
   a.segp = (a.seg + 3) & ~3;
   a.taps_chunk = whole ? whole : 1;
+  if (a.wrow)
+    while (a.kw % a.taps_chunk) --a.taps_chunk;
   a.segs_tap = whole ? 1 : (a.cin + T::kK - 1) / T::kK;
-  a.chunks = cf_chunks(a.cin, taps, PX);
+  a.chunks = whole ? (taps + a.taps_chunk - 1) / a.taps_chunk : taps * a.segs_tap;
   hipLaunchKernelGGL((conv_f32_kernel<PX, CH, VEC>),
                      dim3((unsigned)((a.m + T::kPix - 1) / T::kPix), (unsigned)((a.cout + T::kCh - 1) / T::kCh)),
                      dim3(256), 0, st, a);
@@ -267,10 +270,9 @@ struct CfChoice {
   int px, ch;
   long long wgs;
 };
-CfChoice cf_choose(const DirectArgs& d) {
+CfChoice cf_choose(const DirectArgs& d, int taps) {
   CfChoice best{};
   float least = 0;
-  const int taps = d.kh * d.kw;
   const float kt = (float)taps * (float)d.cin / 64.0f;
   for (int p : {1, 2, 4})
     for (int c : {1, 2, 3, 4, 5}) {
@@ -288,7 +290,31 @@ CfChoice cf_choose(const DirectArgs& d) {
   return best;
 }
 
+// The filter's rows or columns first..last that meet the image of n rows at
+// one of the no outputs at least.
+struct CfSpan {
+  int first, count;
+};
+CfSpan cf_span(int taps, int n, int no, int stride, int pad) {
+  int first = 0, last = -1;
+  for (int k = 0; k < taps; ++k) {
+    const int o = std::max(0, (pad - k + stride - 1) / stride);  // the first output whose tap k is not above the image
+    if (o < no && o * stride - pad + k >= 0 && o * stride - pad + k < n) {
+      if (last < 0) first = k;
+      last = k;
+    }
+  }
+  return last < 0 ? CfSpan{0, 1} : CfSpan{first, last - first + 1};
+}
+
 }  // namespace
+
+// A small map under a large filter: the taps that no output has in its image
+// are cut off (18 maps of one pixel, 47 -> 99 7x7, are a 1x1: 46.9 -> 7 us).
+CfWindow conv_f32_window(const DirectArgs& d) {
+  const CfSpan r = cf_span(d.kh, d.h, d.ho, d.sh, d.pt), c = cf_span(d.kw, d.w, d.wo, d.sw, d.pl);
+  return {r.first, r.count, c.first, c.count};
+}
 
 bool conv_f32_reaches(const DirectArgs& d) {
   // 32-bit byte offsets into the input and the weights, also for the windows
@@ -296,7 +322,7 @@ bool conv_f32_reaches(const DirectArgs& d) {
   const long long xe = ((long long)d.n * d.h * d.w - 1) * d.x_pix_stride + d.cin;
   const long long we = (long long)d.kh * d.kw * d.cin * d.cout;
   const long long edge = ((long long)(d.pt + d.kh + 64) * d.w + d.pl + d.kw) * d.x_pix_stride + 64;
-  const long long wedge = (64ll * d.cin + 64) * d.cout + d.cout;
+  const long long wedge = (64ll * d.cin + 128ll * d.kw + 64) * d.cout + d.cout;
   return d.m > 0 && d.cout <= 8 * 65535 && xe + edge < (1ll << 29) && we + wedge < (1ll << 29);
 }
 
@@ -304,9 +330,9 @@ bool conv_f32_reaches(const DirectArgs& d) {
 // where the tile's per-tap work (a tap is a segment of few steps, kept and put
 // back at the borders) and its eight channels a row of threads weigh: a
 // robust fit (15%) to 627 of them.
-float conv_f32_cost(const DirectArgs& d) {
-  const CfChoice t = cf_choose(d);
-  const int taps = d.kh * d.kw;
+float conv_f32_cost(const DirectArgs& d, const CfWindow& w) {
+  const int taps = w.kh * w.kw;
+  const CfChoice t = cf_choose(d, taps);
   const float chunks = (float)cf_chunks(d.cin, taps, t.px), segs = cf_taps(d.cin, taps, t.px) ? (float)taps : chunks;
   const float kt = (float)taps * (float)d.cin / 64.0f, pc = (float)(t.px * t.ch);
   const float mean = (float)t.wgs / 256.0f, full = (float)((t.wgs + 255) / 256);
@@ -318,19 +344,24 @@ void launch_conv_f32(hipStream_t st, const DirectArgs& d) {
   if (d.in_kind != 0 || d.out_kind != 0 || !conv_f32_reaches(d)) fail(-4, "conv_f32: not a problem of this kernel");
   const long long xe = ((long long)d.n * d.h * d.w - 1) * d.x_pix_stride + d.cin;
   const long long we = (long long)d.kh * d.kw * d.cin * d.cout;
+  const CfWindow win = conv_f32_window(d);
+  const long long wc = (long long)d.cin * d.cout, w0 = (win.kh0 * d.kw + win.kw0) * wc;
   CfArgs a{};
   a.x = (const float*)d.x + d.x_c_off;
-  a.w = d.wf;
+  a.w = d.wf + w0;
+  // one column: its taps are as far apart as rows; several: a chunk stays in a row
+  a.wtap = (int)((win.kw == 1 ? d.kw : 1) * wc);
+  a.wrow = (int)(win.kw == 1 || win.kh == 1 ? 0 : (d.kw - win.kw) * wc);
   a.bias = d.bias_f;
   a.y = (float*)d.y + d.y_c_off;
-  a.n = d.n; a.h = d.h; a.wd = d.w; a.cin = d.cin; a.cout = d.cout; a.kh = d.kh; a.kw = d.kw;
-  a.sh = d.sh; a.sw = d.sw; a.pt = d.pt; a.pl = d.pl; a.ho = d.ho; a.wo = d.wo; a.m = d.m;
+  a.n = d.n; a.h = d.h; a.wd = d.w; a.cin = d.cin; a.cout = d.cout; a.kh = win.kh; a.kw = win.kw;
+  a.sh = d.sh; a.sw = d.sw; a.pt = d.pt - win.kh0; a.pl = d.pl - win.kw0; a.ho = d.ho; a.wo = d.wo; a.m = d.m;
   a.xs = d.x_pix_stride;
   a.ys = d.y_pix_stride;
   a.act = d.act;
   a.x_bytes = (int)(xe * 4);
-  a.w_bytes = (int)(we * 4);
-  const auto [px, ch, wgs] = cf_choose(d);
+  a.w_bytes = (int)((we - w0) * 4);
+  const auto [px, ch, wgs] = cf_choose(d, win.kh * win.kw);
   const bool vec = d.cin % 4 == 0 && d.x_pix_stride % 4 == 0 && (uintptr_t)a.x % 16 == 0;
 #define DW_CF(P, C) \
   if (px == P && ch == C) vec ? launch_tile<P, C, true>(st, a) : launch_tile<P, C, false>(st, a);

@@ -675,7 +675,8 @@ int direct_channels(const DirectArgs& a, bool vin) {
 bool conv_f32_tiles(const DirectArgs& a) {
   if (a.in_kind != 0 || a.out_kind != 0 || !conv_f32_reaches(a)) return false;
   if (a.cin > 24 && a.cout > 4) return true;
-  const float taps = (float)(a.kh * a.kw), K = taps * (float)a.cin;
+  const CfWindow win = conv_f32_window(a);
+  const float taps = (float)(win.kh * win.kw), K = taps * (float)a.cin;
   const bool vin = vec_in(a);
   const int c1 = conv1x1_exact_channels(a), c = c1 ? c1 : direct_channels(a, vin);
   const long waves = ((long)a.m + 63) / 64 * (a.cout / c);
@@ -685,7 +686,7 @@ bool conv_f32_tiles(const DirectArgs& a) {
                                    0.000245f * g * K * o
                              : 3.61f + 0.0253f * taps + K * (0.0336f + 0.00249f * o) + 0.0406f * full * K +
                                    0.132f * g * o;
-  return direct >= 1.2f * conv_f32_cost(a);
+  return direct >= 1.2f * conv_f32_cost(a, win);
 }
 
 void launch_direct_conv(hipStream_t st, const DirectArgs& a_in) {

@@ -107,6 +107,43 @@ def test_conv_f32_of_few_channels(backend, x_shape, w_shape, s, limit):
     assert t < limit * relu_time(backend, max(x.size, want.size))
 
 
+# every tap of the filter on maps that few of them meet: 13, 6, 6 and 10 times as long as the relu
+@pytest.mark.parametrize("x_shape,w_shape,s,limit", [
+    ((18, 1, 1, 47), (7, 7, 47, 99), 1, 5),      # one tap
+    ((11, 1, 23, 20), (7, 7, 20, 1), 1, 4),      # one row
+    ((14, 40, 1, 20), (7, 7, 20, 40), 1, 6),     # one column
+    ((5, 2, 2, 28), (7, 7, 28, 4), 1, 5),        # three rows of three, several taps a chunk
+])
+def test_conv_f32_of_taps_outside_the_image(backend, x_shape, w_shape, s, limit):
+    test_conv_f32_of_few_channels(backend, x_shape, w_shape, s, limit)
+
+
+# the same cuts where the register-tiled kernel takes them: whole taps and parts of taps a chunk, strides that
+# leave taps between unmet, infinite weights in the taps that are cut off
+@pytest.mark.parametrize("x_shape,w_shape,s", [
+    ((9, 2, 3, 12), (7, 5, 12, 40), 1), ((23, 7, 2, 188), (7, 7, 188, 13), 2), ((3, 1, 5, 40), (5, 9, 40, 33), 2),
+    ((4, 6, 1, 300), (9, 7, 300, 20), 3), ((2, 1, 1, 16), (3, 3, 16, 24), 2), ((2, 3, 3, 30), (9, 9, 30, 9), 4),
+])
+def test_conv_f32_cut_filters(backend, x_shape, w_shape, s):
+    r = np.random.default_rng(sum(x_shape))
+    (n, h, w, ci), (kh, kw, _, co) = x_shape, w_shape
+    ph, pw = kh // 2, kw // 2
+    x, wt = r.uniform(-1, 1, x_shape).astype(np.float32), r.uniform(-1, 1, w_shape).astype(np.float32)
+    ho, wo = oracle.out_hw(h, w, kh, kw, s, s, ph, pw)
+    rows = [k for k in range(kh) if any(0 <= o * s - ph + k < h for o in range(ho))]
+    cols = [k for k in range(kw) if any(0 <= o * s - pw + k < w for o in range(wo))]
+    unmet = np.ones((kh, kw), bool)
+    unmet[np.ix_(rows, cols)] = False
+    assert unmet.any()
+    wt[unmet] = np.inf
+    want = oracle.conv2d_f32_nhwc(x, wt, (s, s), (ph, pw))
+    assert np.isfinite(want).all()
+    by = backend.alloc(want.nbytes)
+    ops.conv2d_bias_act_f32_nhwc(backend, backend.from_numpy(x), backend.from_numpy(wt), None, by, n, h, w, ci, co, kh,
+                                 kw, s, s, ph, pw)
+    np.testing.assert_array_equal(backend.to_numpy(by, np.float32, want.shape), want)
+
+
 @pytest.mark.parametrize("x_shape,w_shape", [
     # few channels on the side of the rule that keeps the tiles: odd quads of K and several taps a chunk
     ((1, 20, 21, 13), (5, 5, 13, 17)), ((2, 31, 33, 3), (7, 7, 3, 101)), ((4, 40, 41, 7), (3, 3, 7, 70)),
