@@ -203,6 +203,29 @@ def test_quantized_pool_of_few_pixels(backend, n, h, w, c):
     np.testing.assert_array_equal(backend.to_numpy(by, np.uint8, (n, c)), oracle.qlinear_gap_u8(x, 0.03, 125, 0.01, 128))
 
 
+# four columns of outputs a thread, whatever the map's width: 1.4 and 1.7 times as long as the map on its side (f16)
+@pytest.mark.parametrize("shape,s", [((32, 200, 1, 512), 2), ((26, 58, 2, 712), 2), ((19, 126, 1, 136), 1), ((3, 7, 2, 24), 2),
+                                     ((2, 5, 1, 8), 1), ((40, 200, 2, 256), 1)])
+@pytest.mark.parametrize("f16", [False, True])
+def test_depthwise_of_narrow_maps(backend, shape, s, f16):
+    n, h, w, c = shape
+    r = np.random.default_rng(c)
+    x, k = r.uniform(-1, 1, shape).astype(np.float32), r.uniform(-1, 1, (3, 3, c)).astype(np.float32)
+    fn, ref = ops.depthwise_conv2d_f32_nhwc, oracle.depthwise_f32
+    if f16:
+        x, k = x.astype(np.float16).view(np.uint16), k.astype(np.float16).view(np.uint16)
+        fn, ref = ops.depthwise_conv2d_f16_nhwc, oracle.depthwise_fp16
+    bx, bk = backend.from_numpy(x), backend.from_numpy(k)
+    want = ref(x, k, (s, s), (1, 1))
+    by = backend.alloc(want.nbytes)
+    if f16 and n > 20 and s == 2:
+        t = [per_call(backend, lambda: fn(backend, bx, bk, None, by, n, hh, ww, c, 3, 3, s, s, 1, 1))
+             for hh, ww in ((w, h), (h, w))]
+        assert t[1] < 1.2 * t[0]
+    fn(backend, bx, bk, None, by, n, h, w, c, 3, 3, s, s, 1, 1)
+    np.testing.assert_array_equal(backend.to_numpy(by, x.dtype, want.shape), want)
+
+
 # in tiles of 64 anchors with the loads of 160 channels: 46 and 4.5 times as long as the relu
 @pytest.mark.parametrize("f16", [False, True])
 @pytest.mark.parametrize("n,hw,nc,reg_max,limit", [(20000, [(1, 2), (1, 1)], 2, 2, 12),
