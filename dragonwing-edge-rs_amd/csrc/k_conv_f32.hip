@@ -43,7 +43,7 @@ struct CfArgs {
   int taps_chunk;  // segments in a chunk
   int segs_tap;    // segments of a tap (1 if whole taps fit)
   int chunks;
-  int wtap, wrow;  // weights between two taps, and more between two rows of them
+  int wtap, wrow;  // rows of the weights between two taps, and more between two rows of taps
   int act;
   int x_bytes, w_bytes;
 };
@@ -70,8 +70,9 @@ struct CfTile {
 };
 
 // VEC: c_in % 4 == 0 and 16-byte aligned pixels, so the input comes in four
-// channels at a time.
-template <int PX, int CH, bool VEC>
+// channels at a time.  CUT: columns of the filter are left out between its rows
+// (a test of it a chunk costs the other layers 1%).
+template <int PX, int CH, bool VEC, bool CUT>
 __global__ __launch_bounds__(256, (CfTile<PX, CH, VEC>::kWaves)) void conv_f32_kernel(const CfArgs a) {
   using T = CfTile<PX, CH, VEC>;
   constexpr int K = T::kK, LD = T::kLd, V = T::kV;
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(256, (CfTile<PX, CH, VEC>::kWaves)) void conv_f32_k
 #pragma unroll
   for (int i = 0; i < T::kWLoads; ++i) {
     const int idx = t + 256 * i, k = idx / T::kCh, tl = k / a.segp;
-    wo[i] = tl * a.wtap + (k - tl * a.segp) * a.cout + c0 + idx % T::kCh;
+    wo[i] = (tl * a.wtap + k - tl * a.segp) * a.cout + c0 + idx % T::kCh;
   }
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, a.x_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)a.w, (short)0, a.w_bytes, 0x00020000);
@@ -117,7 +118,7 @@ __global__ __launch_bounds__(256, (CfTile<PX, CH, VEC>::kWaves)) void conv_f32_k
     const int tap = tap0 + ktl;
     const int kh = tap / a.kw, kw = tap - kh * a.kw;
     const int koff = (kh * a.wd + kw) * a.xs + ic0 + kic;
-    const int woff = tap0 * a.wtap + tap0 / a.kw * a.wrow + ic0 * a.cout;
+    const int woff = (tap0 * a.wtap + ic0 + (CUT ? tap0 / a.kw * a.wrow : 0)) * a.cout;
 #pragma unroll
     for (int i = 0; i < T::kXLoads; ++i) {
       if constexpr (VEC)
@@ -239,18 +240,18 @@ __global__ __launch_bounds__(256, (CfTile<PX, CH, VEC>::kWaves)) void conv_f32_k
   }
 }
 
-template <int PX, int CH, bool VEC>
+template <int PX, int CH, bool VEC, bool CUT = false>
 void launch_tile(hipStream_t st, CfArgs a) {
   using T = CfTile<PX, CH, VEC>;
   const int taps = a.kh * a.kw, whole = cf_taps(a.cin, taps, PX);
   a.seg = whole ? a.cin : T::kK;
   a.segp = (a.seg + 3) & ~3;
   a.taps_chunk = whole ? whole : 1;
-  if (a.wrow)
+  if (CUT)
     while (a.kw % a.taps_chunk) --a.taps_chunk;
   a.segs_tap = whole ? 1 : (a.cin + T::kK - 1) / T::kK;
   a.chunks = whole ? (taps + a.taps_chunk - 1) / a.taps_chunk : taps * a.segs_tap;
-  hipLaunchKernelGGL((conv_f32_kernel<PX, CH, VEC>),
+  hipLaunchKernelGGL((conv_f32_kernel<PX, CH, VEC, CUT>),
                      dim3((unsigned)((a.m + T::kPix - 1) / T::kPix), (unsigned)((a.cout + T::kCh - 1) / T::kCh)),
                      dim3(256), 0, st, a);
   DW_HIP(hipGetLastError());
@@ -266,17 +267,20 @@ void launch_tile(hipStream_t st, CfArgs a) {
 // and long chunks on few pixels (20 x 20, 128 -> 128: 18.5 us at 1 x 1
 // against 46.7 us at 2 x 4, with a repacking launch that is gone), FMAs per LDS read for large ones on many (16
 // x 80 x 80, 64 -> 64: 140 us at 4 x 4 against 243 us at 1 x 2).
+bool cf_cut(const DirectArgs& d, const CfWindow& win) { return win.kw > 1 && win.kh > 1 && win.kw < d.kw; }
 struct CfChoice {
   int px, ch;
   long long wgs;
 };
-CfChoice cf_choose(const DirectArgs& d, int taps) {
+// Cut filters take tiles of one pixel a thread: their maps are small.
+CfChoice cf_choose(const DirectArgs& d, const CfWindow& win) {
+  const int taps = win.kh * win.kw;
   CfChoice best{};
   float least = 0;
   const float kt = (float)taps * (float)d.cin / 64.0f;
   for (int p : {1, 2, 4})
     for (int c : {1, 2, 3, 4, 5}) {
-      if (c == 1 && p > 1) continue;
+      if ((c == 1 || cf_cut(d, win)) && p > 1) continue;
       const long long wgs = (((long long)d.m + 32 * p - 1) / (32 * p)) * ((d.cout + 8 * c - 1) / (8 * c));
       const float mean = (float)wgs / 256.0f, full = (float)((wgs + 255) / 256);
       const float chunks = (float)cf_chunks(d.cin, taps, p), fmas = kt * (float)(p * c);
@@ -296,15 +300,14 @@ struct CfSpan {
   int first, count;
 };
 CfSpan cf_span(int taps, int n, int no, int stride, int pad) {
-  int first = 0, last = -1;
-  for (int k = 0; k < taps; ++k) {
+  auto met = [&](int k) {
     const int o = std::max(0, (pad - k + stride - 1) / stride);  // the first output whose tap k is not above the image
-    if (o < no && o * stride - pad + k >= 0 && o * stride - pad + k < n) {
-      if (last < 0) first = k;
-      last = k;
-    }
-  }
-  return last < 0 ? CfSpan{0, 1} : CfSpan{first, last - first + 1};
+    return o < no && o * stride - pad + k >= 0 && o * stride - pad + k < n;
+  };
+  int first = 0, last = taps - 1;
+  while (first < last && !met(first)) ++first;
+  while (first < last && !met(last)) --last;
+  return {first, last - first + 1};
 }
 
 }  // namespace
@@ -332,7 +335,7 @@ bool conv_f32_reaches(const DirectArgs& d) {
 // robust fit (15%) to 627 of them.
 float conv_f32_cost(const DirectArgs& d, const CfWindow& w) {
   const int taps = w.kh * w.kw;
-  const CfChoice t = cf_choose(d, taps);
+  const CfChoice t = cf_choose(d, w);
   const float chunks = (float)cf_chunks(d.cin, taps, t.px), segs = cf_taps(d.cin, taps, t.px) ? (float)taps : chunks;
   const float kt = (float)taps * (float)d.cin / 64.0f, pc = (float)(t.px * t.ch);
   const float mean = (float)t.wgs / 256.0f, full = (float)((t.wgs + 255) / 256);
@@ -350,8 +353,8 @@ void launch_conv_f32(hipStream_t st, const DirectArgs& d) {
   a.x = (const float*)d.x + d.x_c_off;
   a.w = d.wf + w0;
   // one column: its taps are as far apart as rows; several: a chunk stays in a row
-  a.wtap = (int)((win.kw == 1 ? d.kw : 1) * wc);
-  a.wrow = (int)(win.kw == 1 || win.kh == 1 ? 0 : (d.kw - win.kw) * wc);
+  a.wtap = (win.kw == 1 ? d.kw : 1) * d.cin;
+  a.wrow = (d.kw - win.kw) * d.cin;
   a.bias = d.bias_f;
   a.y = (float*)d.y + d.y_c_off;
   a.n = d.n; a.h = d.h; a.wd = d.w; a.cin = d.cin; a.cout = d.cout; a.kh = win.kh; a.kw = win.kw;
@@ -361,8 +364,13 @@ void launch_conv_f32(hipStream_t st, const DirectArgs& d) {
   a.act = d.act;
   a.x_bytes = (int)(xe * 4);
   a.w_bytes = (int)((we - w0) * 4);
-  const auto [px, ch, wgs] = cf_choose(d, win.kh * win.kw);
+  const auto [px, ch, wgs] = cf_choose(d, win);
   const bool vec = d.cin % 4 == 0 && d.x_pix_stride % 4 == 0 && (uintptr_t)a.x % 16 == 0;
+  const bool cut = cf_cut(d, win);
+#define DW_CUT(C) \
+  if (cut && ch == C) return vec ? launch_tile<1, C, true, true>(st, a) : launch_tile<1, C, false, true>(st, a);
+  DW_CUT(1) DW_CUT(2) DW_CUT(3) DW_CUT(4) DW_CUT(5)
+#undef DW_CUT
 #define DW_CF(P, C) \
   if (px == P && ch == C) vec ? launch_tile<P, C, true>(st, a) : launch_tile<P, C, false>(st, a);
   DW_CF(1, 1) DW_CF(1, 2) DW_CF(1, 3) DW_CF(1, 4) DW_CF(1, 5)
