@@ -83,7 +83,8 @@ struct IgemmArgs {
                            // -1: the streamed-weight kernel (long K); -2: the row-tile kernel;
                            // -3: the wide-tile kernel (c_in % 128 == 0); -4 / -5: the
                            // band-tile kernel with 8 / 16 waves (tile_pb: its band height);
-                           // -6: the split-K kernel (tile_pb: its waves)
+                           // -6: the split-K kernel (tile_pb: its waves); -7: the in-order
+                           // fp16 kernel
   int band_rows;           // set by the launcher for the band-tile kernel
   // EPI_QU8 (table or plain requantize epilogues) and EPI_F16: a nearest
   // 2x upsample of the output written as well (the resize folded into its

@@ -1,4 +1,4 @@
-"""Gemm (f32, f16; plain and transposed B) at the edges of its 16 x 16 tiles
+"""Gemm (f32, f16; plain and transposed B) at the edges of its 8 x 16 tiles
 and 256-step chunks of K: every bit equals the oracle's, which walks each sum
 in the reference's order."""
 import numpy as np
@@ -10,7 +10,8 @@ from dragonwing_edge_rs_amd.graph import GRAPH_F16, GRAPH_F32, Graph, HipGraphRu
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 1, 1), (16, 16, 256), (17, 15, 257), (1, 33, 255), (33, 1, 511), (5, 40, 513), (2, 1003, 3), (65, 31, 1030)]
+SHAPES = [(1, 1, 1), (16, 16, 256), (17, 15, 257), (1, 33, 255), (33, 1, 511), (5, 40, 513), (2, 1003, 3), (65, 31, 1030), (7, 16, 300),
+          (8, 17, 256), (9, 15, 258)]
 
 
 @pytest.mark.parametrize("mnk", SHAPES)

@@ -17,9 +17,13 @@ pytestmark = pytest.mark.gpu
     (16, 20, 3),     # K = 144: a partial third k-step; a group of 16 and one quad
     (48, 84, 3),     # K = 432; 96-channel tile
     (128, 36, 3),    # 18 k-steps: more than the 16 waves of a workgroup
-    (16, 896, 1),    # exactly one launch's channels
-    (32, 900, 1),    # one quad past it
-    (16, 1800, 1),   # three launches
+    (16, 896, 1),    # one launch, whole tiles
+    (32, 900, 1),    # one launch, padding channels
+    (16, 1008, 1),   # exactly one launch's channels, the padding's groups with them
+    (48, 1012, 1),   # one quad in a second launch
+    (16, 1800, 1),   # two launches
+    (80, 2016, 1),   # exactly two
+    (16, 2048, 3),   # three, the middle one whole
 ])
 def test_qconv_prep_bit_exact(backend, c_in, c_out, k):
     r = np.random.default_rng(c_in + 7 * c_out + k)
